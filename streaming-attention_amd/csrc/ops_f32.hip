@@ -6,7 +6,10 @@
 // tensor_cpp/src/qwen3_ops.cpp qwen3_mlp :265-296) with fp32 weights, so the
 // layer keeps fp32 arithmetic end to end.  Every operator reads and writes
 // HBM once per element; the linear is the only one with data reuse.
+#include <math.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "sa_internal.h"
 
@@ -24,13 +27,13 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // 64 x 32 blocks of x and w through LDS, k-major, so that a fragment read
 // (lane l: row l & 15 at k = l >> 4) is 16 consecutive floats per k.  Rows,
 // columns and k past the matrix read as zero; stores are bounds-checked.
-// VEC: K % 4 == 0 and 16-byte aligned x and w, so blocks load as float4.
+// For K and pointers that float4 loads cannot take (K % 4 != 0, x or w not
+// 16-byte aligned); the others take linear_f32_direct_kernel.
 // ---------------------------------------------------------------------------
 constexpr int kLinTile = 64;
 constexpr int kLinK = 32;
 constexpr int kLinStride = kLinTile + 4;   // floats per LDS k row
 
-template <bool VEC>
 __device__ __forceinline__ void stage_block(const float* __restrict__ src, int rows, int K, int r0, int k0,
                                             float (*dst)[kLinStride]) {
 #pragma unroll
@@ -41,20 +44,15 @@ __device__ __forceinline__ void stage_block(const float* __restrict__ src, int r
         f32x4_t v = {0.f, 0.f, 0.f, 0.f};
         if (row < rows) {
             const float* p = src + (size_t)row * K + k;
-            if constexpr (VEC) {
-                if (k < K) v = *reinterpret_cast<const f32x4_t*>(p);
-            } else {
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (k + j < K) v[j] = p[j];
-            }
+            for (int j = 0; j < 4; ++j)
+                if (k + j < K) v[j] = p[j];
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) dst[kq + j][r] = v[j];
     }
 }
 
-template <bool VEC>
 __global__ void __launch_bounds__(256)
 linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
                   float* __restrict__ y, int M, int N, int K) {
@@ -71,8 +69,8 @@ linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, cons
         for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     for (int k0 = 0; k0 < K; k0 += kLinK) {
-        stage_block<VEC>(x, M, K, m0, k0, xs);
-        stage_block<VEC>(w, N, K, n0, k0, ws);
+        stage_block(x, M, K, m0, k0, xs);
+        stage_block(w, N, K, n0, k0, ws);
         __syncthreads();
 #pragma unroll
         for (int ks = 0; ks < kLinK; ks += 4) {
@@ -99,6 +97,133 @@ linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, cons
                 const int row = m0 + wm + 16 * i + 4 * kl + r;
                 if (row < M) y[(size_t)row * N + col] = acc[i][j][r] + b;
             }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The same product for K % 4 == 0 and 16-byte aligned x and w, without LDS in
+// the k loop.  A workgroup owns a TM x TN output tile; its W waves each take a
+// contiguous range of the 32-wide k steps for the whole tile and add up in
+// LDS at the end, in wave order.  A lane loads two 16-byte pieces of a row per
+// step (lane (r, g): k0 + 4 g .. + 3 and k0 + 16 + 4 g .. + 3 of row r, a whole
+// 128-byte line per row between them, issued together) and uses element j in
+// MFMA j of the piece: any assignment of the k values to the MFMAs' k slots
+// gives the same sum as long as both operands share it.  kLinRing steps of
+// loads are in flight per wave, all issued unconditionally (steps past the
+// last re-read it), so no wait drains them.  Rows and columns past the matrix
+// re-read the last one; their outputs are not stored.  k past K (a last step
+// that is cut) enters as zero from both operands.
+//
+// Bound: HBM / L2 on w for few rows, fp32 MFMA for many.
+// ---------------------------------------------------------------------------
+constexpr int kLinRing = 2;
+// Cost rule of launch_direct: bytes per cycle a CU loads with 16 rows per
+// 16-lane group (measured: one such 1 KiB wave load per 64 cycles), and cycles
+// a tile costs besides (LDS sum, stores).
+constexpr double kLinLoadBytes = 15, kLinTileCycles = 1000;
+
+template <int TM, int TN, int W>
+__global__ void __launch_bounds__(W * 64)
+linear_f32_direct_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+                         float* __restrict__ y, int M, int N, int K, int vec_out) {
+    constexpr int MB = TM / 16, NB = TN / 16, STRIDE = TN + 4;
+    __shared__ __align__(16) float sh[W][TM][STRIDE];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * TN, m0 = blockIdx.y * TM;
+    const int steps = (K - 1) / 32 + 1;
+    const int s0 = (int)((long long)steps * wave / W), s1 = (int)((long long)steps * (wave + 1) / W);
+
+    f32x4_t acc[MB][NB] = {};
+    if (s0 < s1) {   // wave-uniform
+        const float* xp[MB];
+        const float* wp[NB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) xp[i] = x + (size_t)min(m0 + 16 * i + r, M - 1) * K;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) wp[i] = w + (size_t)min(n0 + 16 * i + r, N - 1) * K;
+        f32x4_t xr[kLinRing][MB][2], wr[kLinRing][NB][2];
+        auto load = [&](int step, int slot) {
+            const int k0 = 32 * min(step, s1 - 1) + 4 * g;
+            const int ka = min(k0, K - 4), kb = min(k0 + 16, K - 4);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                wr[slot][i][0] = *reinterpret_cast<const f32x4_t*>(wp[i] + ka);
+                wr[slot][i][1] = *reinterpret_cast<const f32x4_t*>(wp[i] + kb);
+            }
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                xr[slot][i][0] = *reinterpret_cast<const f32x4_t*>(xp[i] + ka);
+                xr[slot][i][1] = *reinterpret_cast<const f32x4_t*>(xp[i] + kb);
+            }
+        };
+        auto compute = [&](int slot) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int a = 0; a < MB; ++a)
+#pragma unroll
+                        for (int b = 0; b < NB; ++b)
+                            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wr[slot][b][h][j], xr[slot][a][h][j],
+                                                                             acc[a][b], 0, 0, 0);
+        };
+        // A step that runs past K: the lanes whose 4 values lie there hold a
+        // re-read of the row's end instead.
+        auto cut = [&](int step, int slot) {
+            if (32 * step + 32 > K) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool on = 32 * step + 16 * h + 4 * g < K;
+#pragma unroll
+                    for (int i = 0; i < NB; ++i) wr[slot][i][h] = on ? wr[slot][i][h] : f32x4_t{};
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) xr[slot][i][h] = on ? xr[slot][i][h] : f32x4_t{};
+                }
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < kLinRing; ++u) load(s0 + u, u);
+        int s = s0;
+        // Whole groups that end before the wave's last step, so no step of
+        // theirs can run past K.
+        for (; s + kLinRing < s1; s += kLinRing) {
+#pragma unroll
+            for (int u = 0; u < kLinRing; ++u) {
+                compute(u);
+                load(s + kLinRing + u, u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kLinRing; ++u) {
+            if (s + u < s1) {
+                cut(s + u, u);
+                compute(u);
+            }
+        }
+    }
+    // acc[a][b]: element i is row 16 a + r, column 16 b + 4 g + i.
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) *reinterpret_cast<f32x4_t*>(&sh[wave][16 * a + r][16 * b + 4 * g]) = acc[a][b];
+    __syncthreads();
+    for (int e = threadIdx.x; e < TM * TN / 4; e += W * 64) {
+        const int m = e / (TN / 4), n = e % (TN / 4) * 4;
+        if (m0 + m >= M || n0 + n >= N) continue;
+        f32x4_t v = *reinterpret_cast<const f32x4_t*>(&sh[0][m][n]);
+#pragma unroll
+        for (int k = 1; k < W; ++k) v += *reinterpret_cast<const f32x4_t*>(&sh[k][m][n]);
+        float* out = y + (size_t)(m0 + m) * N + n0 + n;
+        if (vec_out) {   // N % 4 == 0: the four columns are all inside
+            if (bias) v += f32x4_t{bias[n0 + n], bias[n0 + n + 1], bias[n0 + n + 2], bias[n0 + n + 3]};
+            *reinterpret_cast<f32x4_t*>(out) = v;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n0 + n + i < N) out[i] = v[i] + (bias ? bias[n0 + n + i] : 0.f);
+        }
     }
 }
 
@@ -141,6 +266,46 @@ axpby_f32_kernel(const float* x, float a, const float* y, float b, size_t n, flo
         out[i] = y ? fmaf(a, x[i], b * y[i]) : a * x[i];
 }
 
+template <int TM, int TN, int W>
+void launch_tile(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, hipStream_t st) {
+    const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
+    hipLaunchKernelGGL((linear_f32_direct_kernel<TM, TN, W>), grid, dim3(W * 64), 0, st, x, w, bias, y, M, N, K,
+                       N % 4 == 0 && aligned16(y) ? 1 : 0);
+}
+
+// The tile with the smallest estimated time per CU: tiles per CU times the
+// larger of a tile's MFMA cycles (its waves share the CU's four SIMDs, 32
+// cycles per 16x16x4) and its load cycles, plus a tile's fixed cycles.
+// Measured (N, K = 3072, 1024; weights rotated over 75 MB), tiles 16x16 /
+// 16x32 / 32x32 / 32x64 / 64x64 against linear_f32_kernel, us: M = 1 4.8 / 6.6
+// / 8.6 / 13.7 / 22.5 against 48; M = 128 24 / 18.5 / 18.7 / 15.7 / 27 against
+// 53; M = 1024 169 / 128 / 101 / 92 / 78 against 80.  N, K = 2048, 6144: M = 1
+// 18 .. 107 against 354, M = 1024 673 .. 222 against 472.
+void launch_direct(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
+                   hipStream_t st) {
+    static constexpr int kTiles[][3] = {{16, 16, 8}, {16, 32, 8}, {32, 32, 8}, {32, 64, 4}, {64, 64, 4}};
+    const long long cus = device_cu_count();
+    int best = 4;
+    double best_t = INFINITY;
+    for (int i = 0; i < 5; ++i) {
+        const long long tm = kTiles[i][0], tn = kTiles[i][1];
+        const long long rows = (M + tm - 1) / tm, cols = (N + tn - 1) / tn;
+        if (i < 4 && (rows > 65535 || cols * kTiles[i][2] * 64 > 0xffffffffLL)) continue;   // grid limits
+        const long long per_cu = (rows * cols + cus - 1) / cus;
+        const double mfma = (double)(tm * tn) / 256 * K / 16 * 32, load = (double)(tm + tn) * K * 4 / kLinLoadBytes;
+        const double both = kTiles[i][2] == 4 ? 0.5 * std::min(mfma, load) : 0.0;   // one wave per SIMD: partly serial
+        const double t = per_cu * (std::max(mfma, load) + both + kLinTileCycles);
+        if (t < best_t) { best = i; best_t = t; }
+    }
+    switch (best) {
+        case 0: return launch_tile<16, 16, 8>(x, w, bias, y, M, N, K, st);
+        case 1: return launch_tile<16, 32, 8>(x, w, bias, y, M, N, K, st);
+        case 2: return launch_tile<32, 32, 8>(x, w, bias, y, M, N, K, st);
+        case 3: return launch_tile<32, 64, 4>(x, w, bias, y, M, N, K, st);
+        default: return launch_tile<64, 64, 4>(x, w, bias, y, M, N, K, st);
+    }
+}
+
 // Enough workgroups to cover n once, at most 8 per CU (grid-stride beyond).
 dim3 elementwise_grid(size_t n) {
     const size_t want = (n + 255) / 256;
@@ -162,10 +327,10 @@ extern "C" sa_status sa_linear_f32(const float* x, int M, int K, const float* w,
     const dim3 grid((N + kLinTile - 1) / kLinTile, (M + kLinTile - 1) / kLinTile);
     if (grid.y > 65535u) return fail(SA_EINVAL, "M too large for one launch");
     hipStream_t st = as_stream(stream);
-    if (K % 4 == 0 && aligned16(x) && aligned16(w))
-        hipLaunchKernelGGL(linear_f32_kernel<true>, grid, dim3(256), 0, st, x, w, bias, y, M, N, K);
+    if (K > 0 && K <= (1 << 30) && K % 4 == 0 && aligned16(x) && aligned16(w))
+        launch_direct(x, w, bias, y, M, N, K, st);
     else
-        hipLaunchKernelGGL(linear_f32_kernel<false>, grid, dim3(256), 0, st, x, w, bias, y, M, N, K);
+        hipLaunchKernelGGL(linear_f32_kernel, grid, dim3(256), 0, st, x, w, bias, y, M, N, K);
     SA_CHECK_LAUNCH();
     return SA_OK;
 }

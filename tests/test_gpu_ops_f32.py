@@ -101,3 +101,36 @@ def test_qk_norm_eps_placement(sa, oracle, synth, eps_outside):
     other = oracle.rms_norm_rows(x, w, 1e-6, not eps_outside)
     near(got, want, eps_outside)
     assert rel_l2(got[3:], other[3:]) > 0.5
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 4, 3), (2, 20, 257), (24, 1028, 3070), (17, 1028, 4100), (33, 516, 6145), (31, 1000, 8190),
+                                   (65, 132, 8200), (300, 2052, 1000), (1000, 96, 3000)])
+def test_linear_tiles_and_remainders(sa, synth, M, K, N):
+    """Every tile of the LDS-free kernel (sizes the cost rule gives each of
+    them on 256 CUs), with ragged rows and columns, k ranges that end inside
+    a 32-wide step, fewer steps than waves, and N that takes scalar stores;
+    the rows around the output stay as they were.  fp32 sums in any order are
+    within the bars above."""
+    x = synth.normal(50, M + K, (M, K))
+    w = synth.normal(51, N + K, (N, K), 0.05)
+    b = synth.normal(52, N, (N,))
+    buf = torch.full((M * N + 64,), 7.0, device="cuda")
+    y = buf[32:32 + M * N].view(M, N)
+    sa.linear(torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda(), torch.from_numpy(b).cuda(), out=y)
+    near(y.cpu().numpy(), x.astype(np.float64) @ w.astype(np.float64).T + b, (M, K, N))
+    assert bool((buf[:32] == 7.0).all()) and bool((buf[32 + M * N:] == 7.0).all())
+
+
+def test_linear_non_finite_inputs_stay_in_their_rows_and_columns(sa, synth):
+    """An infinity or NaN in x reaches its row only, one in w its column only,
+    also where the last row, column or k step is re-read for padding."""
+    M, K, N = 21, 36, 50
+    x, w = synth.normal(53, 1, (M, K)), synth.normal(53, 2, (N, K))
+    x[M - 1, K - 1] = np.inf
+    x[3, 0] = np.nan
+    w[N - 1, K - 1] = np.nan
+    got = sa.linear(torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    near(got[ok], want[ok], "finite part")
