@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "few_rows.h"
 #include "sa_internal.h"
 #include "sa_qwen3.h"
 
@@ -45,6 +46,7 @@ struct sa_qwen3 {
     float* rope_sin = nullptr;
     // activations for max_batch rows
     float* x = nullptr;        // residual stream [B][hidden]
+    float* x2 = nullptr;       // its other copy in few-row steps
     float* h = nullptr;        // normed input of the next projection [B][hidden]
     float* q = nullptr;        // [B][Hq D]
     float* k = nullptr;        // [B][Hkv D]
@@ -54,7 +56,7 @@ struct sa_qwen3 {
     float* act = nullptr;      // [B][intermediate]
     float* part = nullptr;     // split-K partial sums
     float* logits = nullptr;   // [B][vocab]
-    float* am_val = nullptr;   // argmax partials [B][kArgBlocks]
+    float* am_val = nullptr;   // argmax partials [B][max(kArgBlocks, kFewHeadBlocks)]
     int32_t* am_idx = nullptr;
     void* ws = nullptr;        // paged decode workspace (grow-only)
     size_t ws_bytes = 0;
@@ -495,6 +497,14 @@ Shapes shapes_of(const sa_qwen3_desc& d, int cus) {
     return s;
 }
 
+// Floats of a split-K partial buffer for B rows: the widest projection's
+// partials, or a few-row step's q | k | v and its o and down splits.
+size_t part_floats(const Shapes& s, size_t B) {
+    size_t part = std::min<size_t>(B, kFewRows) * (s.Nqkv + 2 * kFewSplit * s.H);
+    for (const Gemm* g : {&s.qkv, &s.o, &s.gate_up, &s.down}) part = std::max(part, (size_t)g->S * B * g->N);
+    return part;
+}
+
 template <class T>
 sa_status dev_alloc(sa_qwen3* m, T** p, size_t count) {
     void* raw = nullptr;
@@ -532,13 +542,28 @@ sa_status grow(void** p, size_t* have, size_t need) {
     return SA_OK;
 }
 
+// Logits of M rows and their greedy tokens: few rows take the streaming head
+// (in may hold the final norm's residual sum), more the tiled GEMM on in.x.
+sa_status head(sa_qwen3* m, const Shapes& s, const FewInput& in, int M, float* logits, int32_t* next,
+               hipStream_t st) {
+    if (few_rows_fit(M, s.H))
+        return few_head(in, M, s.H, m->lm_head, s.V, logits, m->am_val, m->am_idx, next, st);
+    SA_TRY(gemm(in.x, M, m->lm_head, s.lm, logits, st));
+    hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgBlocks, M), dim3(256), 0, st, logits, s.V, m->am_val,
+                       m->am_idx);
+    SA_CHECK_LAUNCH();
+    hipLaunchKernelGGL(argmax_final_kernel, dim3(M), dim3(64), 0, st, m->am_val, m->am_idx, kArgBlocks, next);
+    SA_CHECK_LAUNCH();
+    return SA_OK;
+}
+
 // The second stream, its partial buffer and the ordering events of an
 // interleaved step, made once per model (on the model's device).
-sa_status make_side(sa_qwen3* m, size_t part_floats) {
+sa_status make_side(sa_qwen3* m, size_t part) {
     if (m->side) return SA_OK;
     if (!m->part2) {
         void* p = nullptr;
-        SA_HIP_TRY(hipMalloc(&p, std::max<size_t>(part_floats, 1) * sizeof(float)));
+        SA_HIP_TRY(hipMalloc(&p, std::max<size_t>(part, 1) * sizeof(float)));
         m->allocs.push_back(p);
         m->part2 = static_cast<float*>(p);
     }
@@ -600,15 +625,13 @@ extern "C" sa_status sa_qwen3_create(const sa_qwen3_desc* desc, int max_batch, s
     if ((st = dev_alloc(m, &m->rope_sin, half)) != SA_OK) return cleanup(st);
     if ((st = sa_rope_table_init(m->rope_cos, m->rope_sin, d.max_pos, d.head_dim, d.rope_theta, nullptr)) != SA_OK)
         return cleanup(st);
-    size_t part = 0;
-    for (const Gemm* g : {&s.qkv, &s.o, &s.gate_up, &s.down}) part = std::max(part, (size_t)g->S * B * g->N);
-    if ((st = dev_alloc(m, &m->x, B * H)) != SA_OK || (st = dev_alloc(m, &m->h, B * H)) != SA_OK ||
+    const size_t part = part_floats(s, B), am = B * std::max(kArgBlocks, kFewHeadBlocks);
+    if ((st = dev_alloc(m, &m->x, B * H)) != SA_OK || (st = dev_alloc(m, &m->x2, B * H)) != SA_OK || (st = dev_alloc(m, &m->h, B * H)) != SA_OK ||
         (st = dev_alloc(m, &m->q, B * s.Nq)) != SA_OK || (st = dev_alloc(m, &m->k, B * s.Nk)) != SA_OK ||
         (st = dev_alloc(m, &m->v, B * s.Nk)) != SA_OK || (st = dev_alloc(m, &m->q_rope, B * s.Nq)) != SA_OK ||
         (st = dev_alloc(m, &m->attn, B * s.Nq)) != SA_OK || (st = dev_alloc(m, &m->act, B * s.I)) != SA_OK ||
         (st = dev_alloc(m, &m->part, part)) != SA_OK || (st = dev_alloc(m, &m->logits, B * V)) != SA_OK ||
-        (st = dev_alloc(m, &m->am_val, B * kArgBlocks)) != SA_OK ||
-        (st = dev_alloc(m, &m->am_idx, B * kArgBlocks)) != SA_OK)
+        (st = dev_alloc(m, &m->am_val, am)) != SA_OK || (st = dev_alloc(m, &m->am_idx, am)) != SA_OK)
         return cleanup(st);
     if (hipDeviceSynchronize() != hipSuccess) return cleanup(fail(SA_EHIP, "RoPE table init failed"));
     *out = m;
@@ -805,13 +828,7 @@ extern "C" sa_status sa_qwen3_prefill(sa_qwen3* m, sa_kvcache* cache, const int3
     SA_HIP_TRY(hipMemcpy2DAsync(h_last, (size_t)s.H * sizeof(float), h + (size_t)(L - 1) * s.H,
                                 (size_t)L * s.H * sizeof(float), (size_t)s.H * sizeof(float), batch,
                                 hipMemcpyDeviceToDevice, st));
-    SA_TRY(gemm(h_last, batch, m->lm_head, s.lm, out_logits, st));
-    hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgBlocks, batch), dim3(256), 0, st, out_logits, s.V, m->am_val,
-                       m->am_idx);
-    SA_CHECK_LAUNCH();
-    hipLaunchKernelGGL(argmax_final_kernel, dim3(batch), dim3(64), 0, st, m->am_val, m->am_idx, kArgBlocks,
-                       next_tokens);
-    SA_CHECK_LAUNCH();
+    SA_TRY(head(m, s, {h_last, nullptr, 0, nullptr, 0.f, nullptr}, batch, out_logits, next_tokens, st));
     return sa_kvcache_commit(cache, nullptr, batch, L, stream);
 }
 
@@ -839,9 +856,12 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     const float eps = d.rms_eps;
     const float scale = 1.0f / sqrtf((float)d.head_dim);
     float* out_logits = logits ? logits : m->logits;
+    bool few_head_rows = false;   // the head takes the last layer's residual sum of all rows
 
     // Rows [r0, r0 + n) of the batch on one stream: its own split-K partials
-    // and decode workspace; x, h, attn and act rows at the same offsets.
+    // and decode workspace; x, h, attn and act rows at the same offsets.  At
+    // most kFewRows rows take the few-row launches (few_rows.hip): no norm or
+    // activation launches, the residual stream alternating between x and x2.
     struct Rows {
         int r0, n;
         float* part;
@@ -849,10 +869,24 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         size_t ws_bytes;
         hipStream_t st;
         std::vector<int32_t> ids;
+        bool few;
+        float *x, *x_other, *o_part, *down_part;
+    };
+    auto make_rows = [&](int r0, int n, float* part, void* ws, size_t ws_bytes, hipStream_t on) {
+        float* o_part = part + (size_t)n * s.Nqkv;
+        Rows r{r0, n, part, ws, ws_bytes, on, {}, few_rows_fit(n, s.H), m->x + (size_t)r0 * s.H,
+               m->x2 + (size_t)r0 * s.H, o_part, o_part + (size_t)kFewSplit * n * s.H};
+        for (int i = 0; i < n; ++i) r.ids.push_back(r0 + i);
+        return r;
     };
     const int ew_grid_full = std::min(4 * device_cu_count(), (M * s.I / 4 + 255) / 256);
-    auto qkv = [&](const Rows& r, int l) {
-        return gemm(m->h + (size_t)r.r0 * s.H, r.n, m->layers[l].qkv, s.qkv, r.part, r.st);
+    auto qkv = [&](Rows& r, int l) -> sa_status {
+        const sa_qwen3::Layer& L = m->layers[l];
+        if (!r.few) return gemm(m->h + (size_t)r.r0 * s.H, r.n, L.qkv, s.qkv, r.part, r.st);
+        FewInput in{r.x, r.down_part, l ? kFewSplit : 0, L.in_norm, eps, l ? r.x_other : nullptr};
+        SA_TRY(few_project_norm(in, r.n, s.H, L.qkv, s.Nqkv, r.part, r.st));
+        if (l) std::swap(r.x, r.x_other);
+        return SA_OK;
     };
     // The split-K sum of the projection, q/k norm + RoPE, the K/V append and
     // the paged decode in one launch per 64 sequences (plus the LSE merge of
@@ -860,18 +894,33 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     // (A separate split kernel cost 4.7 us per layer.)
     auto attention = [&](const Rows& r, int l) {
         const sa_qwen3::Layer& L = m->layers[l];
-        return sa::append_decode_partials(cache, l, r.part, s.qkv.S, r.n, r.ids.data(), s.Hq, L.q_norm, L.k_norm,
-                                          eps, m->rope_cos, m->rope_sin, d.max_pos, scale,
+        return sa::append_decode_partials(cache, l, r.part, r.few ? 1 : s.qkv.S, r.n, r.ids.data(), s.Hq, L.q_norm,
+                                          L.k_norm, eps, m->rope_cos, m->rope_sin, d.max_pos, scale,
                                           m->attn + (size_t)r.r0 * s.Nq, nullptr, r.ws, r.ws_bytes,
                                           l + 1 == d.num_layers ? 1 : 0, r.st);
     };
-    // o projection, residual + norm, MLP, residual + the next block's norm.
-    auto rest = [&](const Rows& r, int l) -> sa_status {
+    // o projection, residual + norm, MLP, residual + the next block's norm
+    // (few rows: the last two are left to the launch that reads the sum).
+    auto rest = [&](Rows& r, int l) -> sa_status {
         const sa_qwen3::Layer& L = m->layers[l];
+        float* attn = m->attn + (size_t)r.r0 * s.Nq;
         float* x = m->x + (size_t)r.r0 * s.H;
         float* h = m->h + (size_t)r.r0 * s.H;
         float* act = m->act + (size_t)r.r0 * s.I;
-        SA_TRY(gemm(m->attn + (size_t)r.r0 * s.Nq, r.n, L.o, s.o, r.part, r.st));
+        const float* next_norm = l + 1 < d.num_layers ? m->layers[l + 1].in_norm : m->final_norm;
+        if (r.few) {
+            SA_TRY(few_project_split(attn, r.n, s.Nq, L.o, s.H, r.o_part, r.st));
+            FewInput in{r.x, r.o_part, kFewSplit, L.post_norm, eps, r.x_other};
+            SA_TRY(few_gate_up(in, r.n, s.H, L.gate_up, s.I, act, r.st));
+            std::swap(r.x, r.x_other);
+            SA_TRY(few_project_split(act, r.n, s.I, L.down, s.H, r.down_part, r.st));
+            if (l + 1 < d.num_layers || few_head_rows) return SA_OK;
+            hipLaunchKernelGGL(residual_norm_kernel, dim3(r.n), dim3(256), 0, r.st, r.down_part, kFewSplit, r.n, s.H,
+                               r.x, next_norm, eps, h);
+            SA_CHECK_LAUNCH();
+            return SA_OK;
+        }
+        SA_TRY(gemm(attn, r.n, L.o, s.o, r.part, r.st));
         hipLaunchKernelGGL(residual_norm_kernel, dim3(r.n), dim3(256), 0, r.st, r.part, s.o.S, r.n, s.H, x,
                            L.post_norm, eps, h);
         SA_CHECK_LAUNCH();
@@ -880,7 +929,6 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         hipLaunchKernelGGL(swiglu_kernel, dim3(ew_grid), dim3(256), 0, r.st, r.part, s.gate_up.S, r.n, s.I, act);
         SA_CHECK_LAUNCH();
         SA_TRY(gemm(act, r.n, L.down, s.down, r.part, r.st));
-        const float* next_norm = l + 1 < d.num_layers ? m->layers[l + 1].in_norm : m->final_norm;
         hipLaunchKernelGGL(residual_norm_kernel, dim3(r.n), dim3(256), 0, r.st, r.part, s.down.S, r.n, s.H, x,
                            next_norm, eps, h);
         SA_CHECK_LAUNCH();
@@ -910,25 +958,21 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     const long long attn_bytes = total * d.n_kv_heads * d.head_dim * 2LL * kv_elem;
     const char* fenv = std::getenv("SA_DECODE_INTERLEAVE");
     const bool interleave = M >= 2 && (fenv ? std::atoi(fenv) != 0 : attn_bytes >= kInterleaveBytes);
+    Rows all = make_rows(0, M, m->part, m->ws, m->ws_bytes, st);
+    few_head_rows = all.few && !interleave;
     if (!interleave) {
-        Rows all{0, M, m->part, m->ws, m->ws_bytes, st, {}};
-        for (int i = 0; i < M; ++i) all.ids.push_back(i);
         for (int l = 0; l < d.num_layers; ++l) {
             SA_TRY(qkv(all, l));
             SA_TRY(attention(all, l));
             SA_TRY(rest(all, l));
         }
     } else {
-        size_t part_floats = 0;
-        for (const Gemm* g : {&s.qkv, &s.o, &s.gate_up, &s.down})
-            part_floats = std::max(part_floats, (size_t)g->S * m->max_batch * g->N);
-        SA_TRY(make_side(m, part_floats));
+        SA_TRY(make_side(m, part_floats(s, m->max_batch)));
         SA_TRY(grow(&m->ws2, &m->ws2_bytes, need));
         int cut = 1;
         while (cut < M - 1 && 2 * prefix[cut] < total) ++cut;
-        Rows a{0, cut, m->part, m->ws, m->ws_bytes, st, {}};
-        Rows b{cut, M - cut, m->part2, m->ws2, m->ws2_bytes, m->side, {}};
-        for (int i = 0; i < M; ++i) (i < cut ? a.ids : b.ids).push_back(i);
+        Rows a = make_rows(0, cut, m->part, m->ws, m->ws_bytes, st);
+        Rows b = make_rows(cut, M - cut, m->part2, m->ws2, m->ws2_bytes, m->side);
         hipEvent_t fork = m->events[0], join = m->events[1], a_first = m->events[2];
         SA_HIP_TRY(hipEventRecord(fork, st));
         SA_HIP_TRY(hipStreamWaitEvent(m->side, fork, 0));
@@ -954,13 +998,9 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         SA_HIP_TRY(hipStreamWaitEvent(st, join, 0));
         if (ls != SA_OK) return ls;
     }
-    // ---- final norm (folded above), lm_head, greedy argmax ----
-    SA_TRY(gemm(m->h, M, m->lm_head, s.lm, out_logits, st));
-    hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgBlocks, M), dim3(256), 0, st, out_logits, s.V, m->am_val,
-                       m->am_idx);
-    SA_CHECK_LAUNCH();
-    hipLaunchKernelGGL(argmax_final_kernel, dim3(M), dim3(64), 0, st, m->am_val, m->am_idx, kArgBlocks,
-                       next_tokens);
-    SA_CHECK_LAUNCH();
+    // ---- final norm, lm_head, greedy argmax ----
+    FewInput last{m->h, nullptr, 0, nullptr, 0.f, nullptr};   // normed by the last layer's residual launch
+    if (few_head_rows) last = {all.x, all.down_part, kFewSplit, m->final_norm, eps, nullptr};
+    SA_TRY(head(m, s, last, M, out_logits, next_tokens, st));
     return SA_OK;   // the last layer's sa_append_decode committed the token
 }

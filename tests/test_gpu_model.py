@@ -270,3 +270,21 @@ def test_model_decode_interleaved_graph_replay(sa, synth, monkeypatch):
     del graph
     cache.close()
     model.close()
+
+
+@pytest.mark.parametrize("rows,hidden,intermediate,vocab", [
+    (1, 1536, 96, 1088), (2, 256, 544, 64), (3, 512, 160, 4160), (5, 256, 512, 1024), (8, 768, 32, 1024),
+    (9, 1024, 224, 1088), (16, 512, 3072, 1024), (17, 256, 512, 1024), (4, 320, 512, 1024), (2, 1792, 64, 128)])
+def test_model_decode_few_rows(sa, oracle, synth, interleave, rows, hidden, intermediate, vocab):
+    """Row counts and shapes at the edges of the few-row launches (1 .. 16 rows
+    by row pairs, hidden a multiple of 256 up to 1536; k ranges of waves that
+    are short, ragged or empty) and just outside them, at the fp32 bar."""
+    cfg = dict(SMALL, hidden=hidden, intermediate=intermediate, vocab=vocab, head_dim=64 if rows % 2 else 128)
+
+    def check(t, got, want):
+        assert np.abs(got - want).max() <= 1e-4 * max(1.0, float(np.abs(want).max()) / 10), f"step {t}"
+        assert rel_l2(got, want) <= 1e-5, f"step {t}"
+
+    lens = [1 + (37 * i) % 150 for i in range(rows)]
+    run_parity(sa, oracle, synth, cfg, 0.05, lens, 3, sa.SA_DTYPE_F32, 60 + rows,
+               [(11 * i + 3) % vocab for i in range(rows)], check)
