@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "few_rows.h"
+#include "proj.h"
 #include "sa_internal.h"
 #include "sa_qwen3.h"
 
@@ -431,15 +432,13 @@ __global__ void argmax_final_kernel(const float* pv, const int32_t* pi, int nb, 
 // ---------------------------------------------------------------------------
 // Host helpers
 // ---------------------------------------------------------------------------
-// Split-K count for an M-row projection: doubled while the grid has fewer
-// than two workgroups per CU, each split keeping at least min_steps k-steps
-// and the partials at most max_cols * M floats (the partial buffer).
-int pick_split(int N, int K, int cus, int M = kMaxRows, int min_steps = 2, long long max_cols = 1LL << 30,
-               int cw = 1) {
-    const int nb = N / (kGN * cw), chunks = K / kGK, mt = (M + kMaxRows - 1) / kMaxRows;
+// Split-K count of a decode step's projection (one row tile): doubled while the
+// grid has fewer than two workgroups per CU, each split keeping at least
+// min_steps k-steps.
+int pick_split(int N, int K, int cus, int min_steps) {
+    const int nb = N / kGN, chunks = K / kGK;
     int s = 1;
-    while (s * 2 <= 32 && (long long)nb * s * mt < 2LL * cus && chunks % (s * 2) == 0 &&
-           chunks / (s * 2) >= min_steps && (long long)N * s * 2 <= max_cols)
+    while (s * 2 <= 32 && (long long)nb * s < 2LL * cus && chunks % (s * 2) == 0 && chunks / (s * 2) >= min_steps)
         s *= 2;
     return s;
 }
@@ -486,11 +485,11 @@ Shapes shapes_of(const sa_qwen3_desc& d, int cus) {
     // 20.76 / 20.78 / 21.00 ms on one box.  128-column workgroups for qkv
     // and gate_up measured slower (20.72 ms, 20.79 with 4-step splits,
     // against 20.67 ms on another box).
-    s.qkv = {s.Nqkv, s.H, pick_split(s.Nqkv, s.H, cus, kMaxRows, 8)};
+    s.qkv = {s.Nqkv, s.H, pick_split(s.Nqkv, s.H, cus, 8)};
     const int od_steps = 4;
-    s.o = {s.H, s.Nq, pick_split(s.H, s.Nq, cus, kMaxRows, od_steps)};
-    s.gate_up = {2 * s.I, s.H, pick_split(2 * s.I, s.H, cus, kMaxRows, 8)};
-    s.down = {s.H, s.I, pick_split(s.H, s.I, cus, kMaxRows, od_steps)};
+    s.o = {s.H, s.Nq, pick_split(s.H, s.Nq, cus, od_steps)};
+    s.gate_up = {2 * s.I, s.H, pick_split(2 * s.I, s.H, cus, 8)};
+    s.down = {s.H, s.I, pick_split(s.H, s.I, cus, od_steps)};
     // lm_head: 128-column workgroups halve the activation re-reads; at
     // vocab 151936, 64 rows: 93.7 us against 111 us per call.
     s.lm = {s.V, s.H, 1, s.V % (2 * kGN) == 0 ? 2 : 1};
@@ -708,8 +707,7 @@ extern "C" sa_status sa_qwen3_init_random(sa_qwen3* m, uint64_t seed, float stde
 
 // A prompt of L tokens for each of sequences 0 .. batch-1 (all empty), run
 // as one causal prefill: the activations are batch * L token rows, the
-// projections the same GEMMs over row tiles (split-K where the column tiles
-// are few), the attention
+// projections GEMMs over row tiles (proj.hip; split-K where the tiles are few), the attention
 // block q/k RMSNorm + RoPE at positions 0 .. L-1, the K/V append, and the
 // causal prefill kernel over the dense token-major q/k/v.  Reference:
 // qwen3_forward_with_cache with an empty cache and S = L
@@ -739,29 +737,17 @@ extern "C" sa_status sa_qwen3_prefill(sa_qwen3* m, sa_kvcache* cache, const int3
     const long long M = (long long)batch * L;
     if (M > 0x7fffffffLL / std::max({s.Nqkv, 2 * s.I, s.H}))
         return fail(SA_ERANGE, "batch * prompt too large");
-    // Split-K only where the row tiles alone leave CUs idle (o_proj and down
-    // at hidden 1024: 16 column tiles; measured for a 512-token prompt at the
-    // Qwen3-0.6B shape, 61.7 us per call unsplit), with at least 8 k-steps
-    // per split and the partials within the qkv / gate_up width.
+    // K splits while the partial sums fit the widest projection's outputs.
     const int cus = device_cu_count();
     const long long part_cols = std::max({s.Nqkv, 2 * s.I, s.H});
     const int m_rows = (int)std::min<long long>(M, 0x7fffffff);
-    // 128-column workgroups (each X fragment read from LDS feeds two MFMAs)
-    // for prompts of more than four 64-row blocks, 64 columns below.
-    // Measured at the Qwen3-0.6B shape through benchmark_qwen3 (tok/s, same
-    // box, interleaved; 64 / 128 columns): 128 tokens 42,100 / 35,900, 256:
-    // 73,200 / 67,200, 384: 88,000 / 89,700, 512: 107,800 / 111,500, 1024:
-    // 128,100 / 141,100, 2048: 118,800 / 133,300.  Shorter prompts give
-    // 128-column grids too few workgroups once split-K keeps its minimum
-    // k-steps per split.
-    auto shape = [&](int N, int K) {
-        const int cw = m_rows > 4 * kMaxRows && N % (2 * kGN) == 0 ? 2 : 1;
-        return Gemm{N, K, pick_split(N, K, cus, m_rows, 8, part_cols, cw), cw};
+    auto plan = [&](int N, int K, bool pair) {
+        return plan_proj(m_rows, N, K, pair, cus, (int)(part_cols / N));
     };
-    const Gemm g_qkv = shape(s.Nqkv, s.H);
-    const Gemm g_o = shape(s.H, s.Nq);
-    const Gemm g_gu = shape(2 * s.I, s.H);
-    const Gemm g_down = shape(s.H, s.I);
+    const ProjPlan g_qkv = plan(s.Nqkv, s.H, false);
+    const ProjPlan g_o = plan(s.H, s.Nq, false);
+    const ProjPlan g_gu = plan(s.I, s.H, true);
+    const ProjPlan g_down = plan(s.H, s.I, false);
 
     // activations of the M token rows, carved from one grow-only buffer
     const size_t f_x = M * s.H, f_q = M * s.Nq, f_k = M * s.Nk, f_act = M * s.I;
@@ -796,31 +782,28 @@ extern "C" sa_status sa_qwen3_prefill(sa_qwen3* m, sa_kvcache* cache, const int3
     hipLaunchKernelGGL(embed_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, m->embed, tokens, s.V, s.H,
                        m->layers[0].in_norm, eps, x, h);
     SA_CHECK_LAUNCH();
-    const int ew_grid = (int)std::min<long long>(4LL * device_cu_count(), (M * s.I / 4 + 255) / 256);
     const int64_t q_str[3] = {(int64_t)L * s.Nq, s.D, s.Nq};
     const int64_t kv_str[3] = {(int64_t)L * s.Nk, s.D, s.Nk};
     for (int l = 0; l < d.num_layers; ++l) {
         const sa_qwen3::Layer& Ly = m->layers[l];
         // ---- attention block ----
-        SA_TRY(gemm(h, (int)M, Ly.qkv, g_qkv, part, st));
+        SA_TRY(project(h, (int)M, Ly.qkv, g_qkv, part, st));
         // q, k, v summed from the projection's split-K partials, q and k
         // normed and rotated (positions 0 .. L-1: the cache is empty), K and V
         // appended to the cache, q, k, v written for the attention: one launch.
-        SA_TRY(qknorm_rope_append_partials(cache, l, part, g_qkv.S, batch, L, s.Hq, Ly.q_norm, Ly.k_norm, eps,
+        SA_TRY(qknorm_rope_append_partials(cache, l, part, g_qkv.split, batch, L, s.Hq, Ly.q_norm, Ly.k_norm, eps,
                                            m->rope_cos, m->rope_sin, d.max_pos, q, k, v, st));
         SA_TRY(sa_prefill_causal_strided_ws(q, k, v, SA_DTYPE_F32, batch, s.Hq, s.Hkv, L, s.D, q_str, kv_str, q_str,
                                             scale, attn, attn_ws, ws_attn, stream));
-        SA_TRY(gemm(attn, (int)M, Ly.o, g_o, part, st));
-        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g_o.S, (int)M, s.H, x,
+        SA_TRY(project(attn, (int)M, Ly.o, g_o, part, st));
+        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g_o.split, (int)M, s.H, x,
                            Ly.post_norm, eps, h);
         SA_CHECK_LAUNCH();
         // ---- MLP ----
-        SA_TRY(gemm(h, (int)M, Ly.gate_up, g_gu, part, st));
-        hipLaunchKernelGGL(swiglu_kernel, dim3(ew_grid), dim3(256), 0, st, part, g_gu.S, (int)M, s.I, act);
-        SA_CHECK_LAUNCH();
-        SA_TRY(gemm(act, (int)M, Ly.down, g_down, part, st));
+        SA_TRY(project(h, (int)M, Ly.gate_up, g_gu, act, st));
+        SA_TRY(project(act, (int)M, Ly.down, g_down, part, st));
         const float* next_norm = l + 1 < d.num_layers ? m->layers[l + 1].in_norm : m->final_norm;
-        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g_down.S, (int)M, s.H,
+        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g_down.split, (int)M, s.H,
                            x, next_norm, eps, h);
         SA_CHECK_LAUNCH();
     }
