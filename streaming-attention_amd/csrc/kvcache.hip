@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <vector>
 
 struct sa_kvcache {
@@ -100,10 +101,13 @@ sa_status publish_lens(sa_kvcache* c, const int32_t* rows, int n, int val, int a
 sa_status refused(const Verdict& v) { return fail(v.status, v.msg); }
 
 // ---------------------------------------------------------------------------
-// Fused QK-norm + RoPE + append.  One wave per (token, head row): waves
-// [0, n_q) handle query heads, [n_q, n_q + n_kv) handle a key head and its
-// value head.  Lane j holds the rotate-half pairs (i, i + D/2) for
-// i = j, j + 64, ... so RoPE needs no lane exchange.
+// Fused QK-norm + RoPE + append.  A head row (query, key or value) is served by
+// D/8 lanes (16 at most), 16 bytes of each half per lane, so RoPE needs no lane
+// exchange and a wave moves 4 rows of 128 elements per load.
+//
+// Bound: the 21 MB of 1024 tokens (16 query and 8 KV heads of 128, bf16 cache)
+// at HBM rate are 3.3 us of a launch.  Rows of 64 lanes with 4-byte loads took
+// 8.8 us: twice the waves, each with four loads of 256 bytes in flight.
 // ---------------------------------------------------------------------------
 struct AppendArgs {
     const float* q; const float* k; const float* v;
@@ -122,6 +126,7 @@ struct AppendArgs {
     const int32_t* table;
     char* k_pool; char* v_pool;
     int n_q, n_kv, S, max_pages, rope_max_pos;
+    int s0, n_s;               // tokens [s0, s0 + n_s) of the S
     float eps;
 };
 
@@ -140,79 +145,166 @@ qk_norm_rope_kernel(const float* x, int n_rows, const int32_t* pos, const float*
     r.store(y + (size_t)row * D, lane);
 }
 
-template <int D, bool BF16>
-__global__ void __launch_bounds__(256)
-qknorm_rope_append_kernel(AppendArgs a) {
-    constexpr int H = D / 2;
-    constexpr int NP = (H + kWave - 1) / kWave;   // pairs per lane
-    const int lane = threadIdx.x & (kWave - 1);
-    const int row_id = blockIdx.x * 4 + threadIdx.x / kWave;
-    const int s = blockIdx.y;
-    const int i_seq = blockIdx.z;
-    const int n_rows = a.n_q + a.n_kv;
-    if (row_id >= n_rows) return;
-    const bool is_q = row_id < a.n_q;
-    if (is_q && !a.q && !a.part) return;
-    const int head = is_q ? row_id : row_id - a.n_q;
-    const int cache_row = a.rows.row[i_seq];
-    const int pos = a.seq_lens[cache_row] + s;
+// A head row over LANES lanes: lane j holds elements i .. i + 3 and their
+// rotate-half partners i + D/2 .. for i = 4 j + 64 c.  The arithmetic is RowPairs'
+// (the same sums in the same order), so both give the same bits.
+template <int D, bool VEC>
+struct RowQuads {
+    static constexpr int H = D / 2;
+    static constexpr int LANES = (H < kWave ? H : kWave) / 4;
+    static constexpr int NC = (H + kWave - 1) / kWave;
+    float lo[NC][4], hi[NC][4];
 
-    const int nh = is_q ? a.n_q : a.n_kv;
-    const size_t src = (((size_t)i_seq * a.S + s) * nh + head) * D;
-    const float* x = (is_q ? a.q : a.k) + src;
-    const float* w = is_q ? a.wq : a.wk;
-
-    const int part_cols = (a.n_q + 2 * a.n_kv) * D;
-    const size_t part_row = (size_t)(a.part_row0 + i_seq * a.S + s) * part_cols;
-    const size_t part_split = (size_t)a.part_M * part_cols;
-    RowPairs<D> r;
-    if (a.part) r.load_sum(a.part + part_row + (is_q ? head : a.n_q + head) * D, part_split, a.part_S, lane);
-    else r.load(x, lane);
-    if (w) r.rms_norm(w, a.eps, lane);
-    if (a.cos_t && pos < a.rope_max_pos) r.rope(a.cos_t, a.sin_t, pos, lane);
-    if (is_q) {
-        r.store(a.q_out + src, lane);
-        return;
-    }
-    if (a.k_out) r.store(a.k_out + src, lane);
-    const float* lo = r.lo;
-    const float* hi = r.hi;
-    // V as given, or summed from the partials (and written to v_out).
-    RowPairs<D> vr;
-    if (a.part) {
-        vr.load_sum(a.part + part_row + (a.n_q + a.n_kv + head) * D, part_split, a.part_S, lane);
-        if (a.v_out) vr.store(a.v_out + src, lane);
-    } else {
-        vr.load(a.v + src, lane);
-    }
-    // Append K (normed, rotated) and V (as given) at pos.  The host has
-    // checked that every row has a page there; these tests only keep a
-    // device length that disagrees with the host from writing out of bounds.
-    if (pos >= a.max_pages * 64) return;
-    const int page = a.table[(size_t)cache_row * a.max_pages + (pos >> 6)];
-    if (page < 0) return;
-    const size_t row = (((size_t)page * a.n_kv + head) * 64 + (pos & 63)) * D;
+    // 4 floats; VEC: 16-byte aligned.
+    __device__ static __forceinline__ void load4(const float* x, float (&v)[4]) {
+        if constexpr (VEC) {
+            const float4 f = *reinterpret_cast<const float4*>(x);
+            v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+        } else {
 #pragma unroll
-    for (int c = 0; c < NP; ++c) {
-        const int i = lane + c * kWave;
-        if (i < H) {
-            if constexpr (BF16) {
-                uint16_t* kd = reinterpret_cast<uint16_t*>(a.k_pool) + row;
-                uint16_t* vd = reinterpret_cast<uint16_t*>(a.v_pool) + row;
-                kd[i] = f32_to_bf16_rne(lo[c]);
-                kd[i + H] = f32_to_bf16_rne(hi[c]);
-                vd[i] = f32_to_bf16_rne(vr.lo[c]);
-                vd[i + H] = f32_to_bf16_rne(vr.hi[c]);
-            } else {
-                float* kd = reinterpret_cast<float*>(a.k_pool) + row;
-                float* vd = reinterpret_cast<float*>(a.v_pool) + row;
-                kd[i] = lo[c];
-                kd[i + H] = hi[c];
-                vd[i] = vr.lo[c];
-                vd[i + H] = vr.hi[c];
+            for (int e = 0; e < 4; ++e) v[e] = x[e];
+        }
+    }
+    __device__ static __forceinline__ void store4(float* y, const float (&v)[4]) {
+        if constexpr (VEC) {
+            *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = v[e];
+        }
+    }
+    __device__ __forceinline__ void load(const float* x, int j) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            load4(x + 4 * j + kWave * c, lo[c]);
+            load4(x + 4 * j + kWave * c + H, hi[c]);
+        }
+    }
+    // The sum, in split order, of S split-K partial rows x[t * split] ...
+    __device__ __forceinline__ void load_sum(const float* x, size_t split, int S, int j) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) lo[c][e] = hi[c][e] = 0.f;
+#pragma unroll 4
+        for (int t = 0; t < S; ++t) {
+            RowQuads p;
+            p.load(x + t * split, j);
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    lo[c][e] += p.lo[c][e];
+                    hi[c][e] += p.hi[c][e];
+                }
+        }
+    }
+    __device__ __forceinline__ void rms_norm(const float* w, float eps, int j) {
+#pragma clang fp contract(off)
+        RowQuads g;
+        g.load(w, j);
+        float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[e] = fmaf(lo[c][e], lo[c][e], fmaf(hi[c][e], hi[c][e], t[e]));
+        const float ss = group_reduce<OpSum, 1, LANES>((t[0] + t[1]) + (t[2] + t[3]));
+        const float rms = sqrtf(ss / (float)D + eps);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                lo[c][e] = (lo[c][e] / rms) * g.lo[c][e];
+                hi[c][e] = (hi[c][e] / rms) * g.hi[c][e];
+            }
+    }
+    __device__ __forceinline__ void rope(const float* cos_t, const float* sin_t, int pos, int j) {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            float cs[4], sn[4];
+            load4(cos_t + (size_t)pos * H + 4 * j + kWave * c, cs);
+            load4(sin_t + (size_t)pos * H + 4 * j + kWave * c, sn);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float l2 = lo[c][e] * cs[e] - hi[c][e] * sn[e];
+                const float h2 = hi[c][e] * cs[e] + lo[c][e] * sn[e];
+                lo[c][e] = l2;
+                hi[c][e] = h2;
             }
         }
     }
+    __device__ __forceinline__ void store(float* y, int j) const {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            store4(y + 4 * j + kWave * c, lo[c]);
+            store4(y + 4 * j + kWave * c + H, hi[c]);
+        }
+    }
+    // A row of the cache pools, 16-byte aligned.
+    template <bool BF16>
+    __device__ __forceinline__ void store_pool(char* pool, size_t row, int j) const {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const size_t i = row + 4 * j + kWave * c;
+            if constexpr (BF16) {
+                auto put = [&](size_t at, const float (&v)[4]) {
+                    uint32_t b[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        b[e] = f32_to_bf16_rne(v[2 * e]) | (uint32_t)f32_to_bf16_rne(v[2 * e + 1]) << 16;
+                    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(pool) + at) = make_uint2(b[0], b[1]);
+                };
+                put(i, lo[c]);
+                put(i + H, hi[c]);
+            } else {
+                float* d = reinterpret_cast<float*>(pool);
+                *reinterpret_cast<float4*>(d + i) = make_float4(lo[c][0], lo[c][1], lo[c][2], lo[c][3]);
+                *reinterpret_cast<float4*>(d + i + H) = make_float4(hi[c][0], hi[c][1], hi[c][2], hi[c][3]);
+            }
+        }
+    }
+};
+
+// VEC: q, k, v, the partials, weights, tables and outputs are 16-byte aligned.
+template <int D, bool BF16, bool VEC>
+__global__ void __launch_bounds__(256)
+qknorm_rope_append_kernel(AppendArgs a) {
+    using Row = RowQuads<D, VEC>;
+    const int j = threadIdx.x % Row::LANES;
+    const unsigned idx = blockIdx.x * (256u / Row::LANES) + threadIdx.x / Row::LANES;
+    const unsigned per_token = a.n_q + 2 * a.n_kv;
+    const int s = a.s0 + (int)(idx / per_token);
+    const int id = (int)(idx % per_token);   // query heads, key heads, value heads
+    const int i_seq = blockIdx.y;
+    if (s >= a.s0 + a.n_s) return;
+    const bool is_q = id < a.n_q, is_k = !is_q && id < a.n_q + a.n_kv;
+    const int head = is_q ? id : is_k ? id - a.n_q : id - a.n_q - a.n_kv;
+    const size_t token = (size_t)i_seq * a.S + s;
+    const size_t src = (token * (is_q ? a.n_q : a.n_kv) + head) * D;
+    const int cache_row = a.rows.row[i_seq];
+    const int pos = a.seq_lens[cache_row] + s;
+    Row r;
+    if (a.part) {
+        const size_t cols = (size_t)per_token * D;
+        r.load_sum(a.part + (a.part_row0 + token) * cols + (size_t)id * D, (size_t)a.part_M * cols, a.part_S, j);
+    } else {
+        r.load((is_q ? a.q : is_k ? a.k : a.v) + src, j);
+    }
+    // The host has checked that every row has a page there; these tests only
+    // keep a device length that disagrees with the host from writing out of
+    // bounds.  Looked up here, so that its round trip overlaps the others.
+    const bool paged = !is_q && pos < a.max_pages * 64;
+    const int page = paged ? a.table[(size_t)cache_row * a.max_pages + (pos >> 6)] : -1;
+    if (is_q || is_k) {
+        const float* w = is_q ? a.wq : a.wk;
+        if (w) r.rms_norm(w, a.eps, j);
+        if (a.cos_t && pos < a.rope_max_pos) r.rope(a.cos_t, a.sin_t, pos, j);
+    }
+    float* copy = is_q ? a.q_out : is_k ? a.k_out : a.v_out;
+    if (copy) r.store(copy + src, j);
+    if (page < 0) return;
+    r.template store_pool<BF16>(is_k ? a.k_pool : a.v_pool, (((size_t)page * a.n_kv + head) * 64 + (pos & 63)) * D, j);
 }
 
 // Dense copy [n_kv][len][D] of one sequence (fp32 out).
@@ -469,7 +561,7 @@ sa_status append_impl(sa_kvcache* c, int layer, const float* q, const float* k, 
     a.k_pool = k_pool_of(c, layer); a.v_pool = v_pool_of(c, layer);
     a.n_q = q || part ? n_q_heads : 0; a.n_kv = c->desc.num_kv_heads; a.S = S;
     a.max_pages = c->desc.max_pages_per_seq; a.rope_max_pos = rope_max_pos; a.eps = eps;
-    const int rows = a.n_q + a.n_kv;
+    const int rows = a.n_q + 2 * a.n_kv;
     const int D = c->desc.head_dim;
     const bool bf = c->desc.kv_dtype == SA_DTYPE_BF16;
     // Up to kRowsPerLaunch sequences per launch, their cache rows by value.
@@ -483,23 +575,38 @@ sa_status append_impl(sa_kvcache* c, int layer, const float* q, const float* k, 
         a.v = v ? v + (size_t)i0 * S * a.n_kv * D : nullptr;
         a.v_out = v_out ? v_out + (size_t)i0 * S * a.n_kv * D : nullptr;
         a.part_row0 = i0 * S;
-        dim3 grid((rows + 3) / 4, S, m);
-        switch (D) {
-#define SA_APPEND_CASE(DD)                                                                        \
-    case DD:                                                                                      \
-        if (bf) hipLaunchKernelGGL((qknorm_rope_append_kernel<DD, true>), grid, dim3(256), 0, st, a); \
-        else hipLaunchKernelGGL((qknorm_rope_append_kernel<DD, false>), grid, dim3(256), 0, st, a); \
+        bool vec = true;   // the launch's pointers allow 16-byte accesses
+        for (const void* p : std::initializer_list<const void*>{a.q, a.k, a.v, a.part, a.q_out, a.k_out, a.v_out, a.wq,
+                                                                a.wk, a.cos_t, a.sin_t})
+            vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+        // Tokens per launch: row indices and the grid stay within 31 bits.
+        const int step = std::max(1, (1 << 28) / rows);
+        for (a.s0 = 0; a.s0 < S; a.s0 += a.n_s) {
+            a.n_s = std::min(step, S - a.s0);
+            const int lanes = std::min(D / 2, kWave) / 4;
+            const dim3 grid((unsigned)(((long long)rows * a.n_s * lanes + 255) / 256), m);
+            switch (D) {
+#define SA_APPEND_LAUNCH(DD, BB, VV)                                                                               \
+    hipLaunchKernelGGL((qknorm_rope_append_kernel<DD, BB, VV>), grid, dim3(256), 0, st, a)
+#define SA_APPEND_CASE(DD)                                                                                         \
+    case DD:                                                                                                       \
+        if (bf && vec) SA_APPEND_LAUNCH(DD, true, true);                                                           \
+        else if (bf) SA_APPEND_LAUNCH(DD, true, false);                                                            \
+        else if (vec) SA_APPEND_LAUNCH(DD, false, true);                                                           \
+        else SA_APPEND_LAUNCH(DD, false, false);                                                                   \
         break;
-            SA_APPEND_CASE(8)
-            SA_APPEND_CASE(16)
-            SA_APPEND_CASE(32)
-            SA_APPEND_CASE(64)
-            SA_APPEND_CASE(128)
-            SA_APPEND_CASE(256)
+                SA_APPEND_CASE(8)
+                SA_APPEND_CASE(16)
+                SA_APPEND_CASE(32)
+                SA_APPEND_CASE(64)
+                SA_APPEND_CASE(128)
+                SA_APPEND_CASE(256)
 #undef SA_APPEND_CASE
-            default: return fail(SA_EINVAL, "head_dim");
+#undef SA_APPEND_LAUNCH
+                default: return fail(SA_EINVAL, "head_dim");
+            }
+            SA_CHECK_LAUNCH();
         }
-        SA_CHECK_LAUNCH();
     }
     return SA_OK;
 }

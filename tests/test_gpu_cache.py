@@ -510,3 +510,39 @@ def test_cache_on_nonblocking_stream(sa, oracle, synth):
     V = v[0].transpose(1, 0, 2)[None]
     assert_f32(host(out)[0], oracle.decode_gqa(q, K, V, SCALE)[0])
     cache.close()
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("d", [8, 16, 32, 64, 128, 256])
+def test_append_equals_standalone_norm_rope(sa, d, shift, bf16):
+    """A prompt's append over ragged row counts, from 16-byte aligned pointers
+    and from pointers 4 bytes past: the bits of the standalone norm + RoPE."""
+    B, S, hq, hkv, eps = 2, 67, 6, 3, 1e-6
+    gen = torch.Generator(device="cuda").manual_seed(d + shift)
+
+    def rand(*shape):
+        n = int(np.prod(shape))
+        return torch.randn(n + shift, device="cuda", generator=gen)[shift:].view(shape)
+    q, k, v = rand(B, S, hq, d), rand(B, S, hkv, d), rand(B, S, hkv, d)
+    wq, wk = rand(d), rand(d)
+    rope = tuple(rand(S, d // 2).copy_(t) for t in sa.rope_tables(S, d, 1e6))
+    cache = sa.KVCache(1, hkv, d, B, 2, 4, sa.SA_DTYPE_BF16 if bf16 else sa.SA_DTYPE_F32)
+    for s in range(B):
+        cache.set_pages(s, [3 - 2 * s, 2 - 2 * s])
+    q_out = rand(B, S, hq, d)
+    cache.append(0, q, k, v, wq, wk, eps, rope, q_out=q_out)
+    cache.commit(S, n_seqs=B)
+    pos = torch.arange(S, dtype=torch.int32, device="cuda").repeat(B)
+
+    def want(x, w):
+        h = x.shape[2]
+        return sa.qk_norm_rope(x.reshape(-1, d).clone(), pos.repeat_interleave(h), w.clone(), eps,
+                               tuple(t.clone() for t in rope)).view(x.shape)
+    assert torch.equal(q_out, want(q, wq))
+    for s in range(B):
+        ks, vs = cache.gather(0, s, S)
+        for got, ref in ((ks, want(k, wk)[s]), (vs, v[s])):
+            ref = ref.transpose(0, 1)
+            assert torch.equal(got, ref.bfloat16().float() if bf16 else ref)
+    cache.close()
