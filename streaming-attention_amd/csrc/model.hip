@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "bf16_terms.h"
 #include "few_rows.h"
 #include "proj.h"
 #include "sa_internal.h"
@@ -76,10 +77,8 @@ struct sa_qwen3 {
 namespace sa {
 namespace {
 
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
-constexpr int kMaxRows = 64;     // batch rows one GEMM tile covers (more rows: more tiles)
 constexpr int kMaxBatch = 1024;  // decode batch rows per model (activations and logits sized for them)
+constexpr int kMaxRows = 64;     // batch rows one GEMM tile covers (more rows: more tiles)
 constexpr int kGN = 64;          // GEMM output columns per workgroup
 constexpr int kGK = 32;          // GEMM k chunk
 constexpr int kArgBlocks = 64;   // argmax workgroups per row
@@ -162,53 +161,47 @@ embed_norm_kernel(const uint16_t* embed, const int32_t* tokens, int vocab, int H
 }
 
 // ---------------------------------------------------------------------------
-// GEMM: P[s][m][n] = sum over k in split s of X[m][k] * W[n][k].
+// GEMM of a decode step whose projections run beside the other half-batch's
+// attention: P[s][m][n] = sum over k in split s of X[m][k] * W[n][k].
 // X fp32 [M][K], W bf16 [N][K]; N % 64 == 0, split % 32 == 0.
 // Workgroup (x, y, z) owns rows 64 z .. 64 z + 63 (rows past M read as zero),
 // columns 64 x .. 64 x + 63 and split y; wave w computes columns
 // 64 x + 16 w .. + 15 for all 64 rows with v_mfma_f32_16x16x32_bf16.
 //
-// The bf16 MFMA takes fp32 X as kGemmTerms bf16 terms: t_0 = rne(x),
+// The bf16 MFMA takes fp32 X as kTerms bf16 terms: t_0 = rne(x),
 // t_i = rne(x - t_0 - ... - t_{i-1}) (each difference is exact in fp32), so
-// |x - sum t_i| <= 2^-9(kGemmTerms) |x|.  Every product t_i * w is exact in
+// |x - sum t_i| <= 2^-9(kTerms) |x|.  Every product t_i * w is exact in
 // fp32 (the weights are bf16) and accumulates in fp32: the result is the fp32
 // GEMM's to within that truncation of X.  Per 32-wide k step the workgroup
 // converts its 64 x 32 block of X into LDS (double-buffered, one barrier per
 // step); W fragments stream from global memory into registers kGemmRing steps
 // ahead of their use, X blocks kGemmXRing steps ahead; the per-step barrier
-// orders LDS only, so those loads stay in flight across it.  (With
-// __syncthreads, which waits for every outstanding global load, each k-step
-// cost about one memory round trip: 46.7 us per projection for a 512-row
-// prompt at the Qwen3-0.6B shape.)
+// orders LDS only, so those loads stay in flight across it.
+//
+// proj.hip's tiles are faster alone (28 layers, B = 64, 64 - 1024 cached
+// tokens: 2.51 against 2.67 ms), but their 112 KiB of LDS and more leave no room on a CU
+// beside the attention's workgroups; these 30 KiB do, and so fill its
+// bubbles: B = 64, 512 - 16384 tokens 11.4 against 11.9 ms.
 // ---------------------------------------------------------------------------
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-
-constexpr int kGemmTerms = 3;     // bf16 terms of each activation (2^-27 |x| left over)
 constexpr int kGemmRing = 8;      // W fragments in flight per wave (k steps)
 constexpr int kGemmXRing = 4;     // X blocks in flight per thread (k steps); divides kGemmRing
 constexpr int kGemmXStride = kGK + 8;   // bf16 per LDS row of X: conflict-free fragment reads
 
-template <int CW>
 __global__ void __launch_bounds__(256)
 gemm_xwt_kernel(const float* __restrict__ X, int M, int K, const uint16_t* __restrict__ W, int N, int split,
                 float* __restrict__ P) {
-    __shared__ __align__(16) uint16_t Xb[2][kGemmTerms][kMaxRows][kGemmXStride];
+    __shared__ __align__(16) uint16_t Xb[2][kTerms][kMaxRows][kGemmXStride];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r16 = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * kGN * CW + 16 * CW * wave;
+    const int n0 = blockIdx.x * kGN + 16 * wave;
     const int k_begin = blockIdx.y * split;
     const int m0 = blockIdx.z * kMaxRows;
     const int Mt = min(M - m0, kMaxRows);
     const int nsteps = split / kGK;
 
-    // W fragment c of step j (A operand): lane (r16, g) holds
-    // W[n0 + 16 c + r16][k + 8 g .. + 7].
+    // W fragment of step j (A operand): lane (r16, g) holds W[n0 + r16][k + 8 g .. + 7].
     const uint16_t* Wl = W + (size_t)(n0 + r16) * K + k_begin + 8 * g;
-    auto load_w = [&](int j, int c) { return *reinterpret_cast<const bf16x8_t*>(Wl + (size_t)c * 16 * K + j * kGK); };
+    auto load_w = [&](int j) { return *reinterpret_cast<const bf16x8_t*>(Wl + j * kGK); };
     // X block of step j: thread t converts X[m0 + t / 4][k + 8 (t % 4) .. + 7].
     // Rows past M load row M - 1 and are zeroed when converted.  Every load of
     // the loop below is issued unconditionally (steps past the last clamp to
@@ -225,41 +218,28 @@ gemm_xwt_kernel(const float* __restrict__ X, int M, int K, const uint16_t* __res
     auto store_x = [&](int buf, f32x4_t a, f32x4_t b) {
         a = x_on ? a : f32x4_t{};
         b = x_on ? b : f32x4_t{};
-        f32x2_t v[4] = {{a[0], a[1]}, {a[2], a[3]}, {b[0], b[1]}, {b[2], b[3]}};
+        bf16x8_t t[kTerms];
+        split_terms(a, b, t);
 #pragma unroll
-        for (int t = 0; t < kGemmTerms; ++t) {
-            u32x4_t packed;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const bf16x2_t h = __builtin_convertvector(v[e], bf16x2_t);
-                const uint32_t bits = __builtin_bit_cast(uint32_t, h);
-                packed[e] = bits;
-                v[e] -= f32x2_t{bf16_lo(bits), bf16_hi(bits)};
-            }
-            *reinterpret_cast<u32x4_t*>(&Xb[buf][t][xr][xc]) = packed;
-        }
+        for (int i = 0; i < kTerms; ++i) *reinterpret_cast<bf16x8_t*>(&Xb[buf][i][xr][xc]) = t[i];
     };
 
     const int last = nsteps - 1;
-    bf16x8_t ring[kGemmRing][CW];
+    bf16x8_t ring[kGemmRing];
 #pragma unroll
-    for (int u = 0; u < kGemmRing; ++u)
-#pragma unroll
-        for (int c = 0; c < CW; ++c) ring[u][c] = load_w(min(u, last), c);
+    for (int u = 0; u < kGemmRing; ++u) ring[u] = load_w(min(u, last));
     // acc[mt]: element i is row m0 + 16 mt + r16, column n0 + 4 g + i.  Term
     // by term, the four row blocks in turn: consecutive MFMAs write
     // different accumulators (each accumulator still adds its terms in
     // order 0, 1, 2).
-    f32x4_t acc[kMaxRows / 16][CW] = {};
-    auto mfma_step = [&](const bf16x8_t (&wf)[CW], int buf) {
+    f32x4_t acc[kMaxRows / 16] = {};
+    auto mfma_step = [&](bf16x8_t wf, int buf) {
 #pragma unroll
-        for (int t = 0; t < kGemmTerms; ++t)
+        for (int t = 0; t < kTerms; ++t)
 #pragma unroll
             for (int mt = 0; mt < kMaxRows / 16; ++mt) {
                 const bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(&Xb[buf][t][16 * mt + r16][8 * g]);
-#pragma unroll
-                for (int c = 0; c < CW; ++c)
-                    acc[mt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[c], xf, acc[mt][c], 0, 0, 0);
+                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[mt], 0, 0, 0);
             }
     };
     static_assert(kGemmRing % kGemmXRing == 0, "the X ring index follows the unrolled W ring index");
@@ -273,12 +253,8 @@ gemm_xwt_kernel(const float* __restrict__ X, int M, int K, const uint16_t* __res
     // Step j = j0 + u, with u = j % kGemmRing known at compile time.
     auto step = [&](int j, int u) {
         const int buf = u & 1;       // kGemmRing is even, so j & 1 == u & 1
-        bf16x8_t wf[CW];
-#pragma unroll
-        for (int c = 0; c < CW; ++c) {
-            wf[c] = ring[u][c];
-            ring[u][c] = load_w(min(j + kGemmRing, last), c);
-        }
+        const bf16x8_t wf = ring[u];
+        ring[u] = load_w(min(j + kGemmRing, last));
         mfma_step(wf, buf);
         // the other buffer was last read before the previous barrier
         const int nx = (u + 1) % kGemmXRing;
@@ -305,10 +281,7 @@ gemm_xwt_kernel(const float* __restrict__ X, int M, int K, const uint16_t* __res
 #pragma unroll
     for (int mt = 0; mt < kMaxRows / 16; ++mt) {
         const int m = 16 * mt + r16;
-        if (m < Mt) {
-#pragma unroll
-            for (int c = 0; c < CW; ++c) *reinterpret_cast<f32x4_t*>(out + (size_t)m * N + 16 * c) = acc[mt][c];
-        }
+        if (m < Mt) *reinterpret_cast<f32x4_t*>(out + (size_t)m * N) = acc[mt];
     }
 }
 
@@ -432,26 +405,24 @@ __global__ void argmax_final_kernel(const float* pv, const int32_t* pi, int nb, 
 // ---------------------------------------------------------------------------
 // Host helpers
 // ---------------------------------------------------------------------------
-// Split-K count of a decode step's projection (one row tile): doubled while the
-// grid has fewer than two workgroups per CU, each split keeping at least
-// min_steps k-steps.
-int pick_split(int N, int K, int cus, int min_steps) {
+// Split-K count of one row tile: doubled while the grid has fewer than two
+// workgroups per CU, each split keeping at least min_steps k-steps and the
+// partials max_cols columns.
+int pick_split(int N, int K, int cus, int min_steps, size_t max_cols) {
     const int nb = N / kGN, chunks = K / kGK;
     int s = 1;
-    while (s * 2 <= 32 && (long long)nb * s < 2LL * cus && chunks % (s * 2) == 0 && chunks / (s * 2) >= min_steps)
+    while (s * 2 <= 32 && (long long)nb * s < 2LL * cus && chunks % (s * 2) == 0 && chunks / (s * 2) >= min_steps &&
+           (size_t)N * s * 2 <= max_cols)
         s *= 2;
     return s;
 }
 
-// cw: 16-column W fragments per wave (1, or 2 for 128-column workgroups).
-struct Gemm { int N, K, S, cw = 1; };
+// N x K projection in S splits.
+struct Gemm { int N, K, S; };
 
 sa_status gemm(const float* X, int M, const uint16_t* W, const Gemm& g, float* P, hipStream_t st) {
-    const dim3 grid(g.N / (kGN * g.cw), g.S, (M + kMaxRows - 1) / kMaxRows);
-    if (g.cw == 2)
-        hipLaunchKernelGGL(gemm_xwt_kernel<2>, grid, dim3(256), 0, st, X, M, g.K, W, g.N, g.K / g.S, P);
-    else
-        hipLaunchKernelGGL(gemm_xwt_kernel<1>, grid, dim3(256), 0, st, X, M, g.K, W, g.N, g.K / g.S, P);
+    const dim3 grid(g.N / kGN, g.S, (M + kMaxRows - 1) / kMaxRows);
+    hipLaunchKernelGGL(gemm_xwt_kernel, grid, dim3(256), 0, st, X, M, g.K, W, g.N, g.K / g.S, P);
     SA_CHECK_LAUNCH();
     return SA_OK;
 }
@@ -469,39 +440,49 @@ namespace {
 
 struct Shapes {
     int H, I, V, Hq, Hkv, D, Nq, Nk, Nqkv;
-    Gemm qkv, o, gate_up, down, lm;
 };
 
-Shapes shapes_of(const sa_qwen3_desc& d, int cus) {
+Shapes shapes_of(const sa_qwen3_desc& d) {
     Shapes s;
     s.H = d.hidden; s.I = d.intermediate; s.V = d.vocab;
     s.Hq = d.n_q_heads; s.Hkv = d.n_kv_heads; s.D = d.head_dim;
     s.Nq = s.Hq * s.D; s.Nk = s.Hkv * s.D; s.Nqkv = s.Nq + 2 * s.Nk;
-    // Decode-step projections (64 rows per tile): splits of at least 8 k-steps,
-    // 4 for the 1024-column o and down projections (16 column blocks: 256
-    // workgroups instead of 128).  Measured on the 28-layer B = 64 step:
-    // 20.79 ms against 20.98 ms with 2-step splits everywhere (the partials'
-    // traffic outweighed the extra workgroups); o/down at 4 / 8 / 16 steps
-    // 20.76 / 20.78 / 21.00 ms on one box.  128-column workgroups for qkv
-    // and gate_up measured slower (20.72 ms, 20.79 with 4-step splits,
-    // against 20.67 ms on another box).
-    s.qkv = {s.Nqkv, s.H, pick_split(s.Nqkv, s.H, cus, 8)};
-    const int od_steps = 4;
-    s.o = {s.H, s.Nq, pick_split(s.H, s.Nq, cus, od_steps)};
-    s.gate_up = {2 * s.I, s.H, pick_split(2 * s.I, s.H, cus, 8)};
-    s.down = {s.H, s.I, pick_split(s.H, s.I, cus, od_steps)};
-    // lm_head: 128-column workgroups halve the activation re-reads; at
-    // vocab 151936, 64 rows: 93.7 us against 111 us per call.
-    s.lm = {s.V, s.H, 1, s.V % (2 * kGN) == 0 ? 2 : 1};
     return s;
 }
 
-// Floats of a split-K partial buffer for B rows: the widest projection's
-// partials, or a few-row step's q | k | v and its o and down splits.
+// Floats of the partial-sum buffer of a decode step of up to B rows: a
+// few-row step's q | k | v and its o and down splits, or 8 splits of the wider of
+// qkv and o / down for up to 128 rows (more rows take fewer), gate and up unsplit.
 size_t part_floats(const Shapes& s, size_t B) {
-    size_t part = std::min<size_t>(B, kFewRows) * (s.Nqkv + 2 * kFewSplit * s.H);
-    for (const Gemm* g : {&s.qkv, &s.o, &s.gate_up, &s.down}) part = std::max(part, (size_t)g->S * B * g->N);
-    return part;
+    const size_t few = std::min<size_t>(B, kFewRows) * (s.Nqkv + 2 * kFewSplit * s.H);
+    return std::max({few, 8 * std::min<size_t>(B, 128) * std::max(s.Nqkv, s.H), B * std::max({s.Nqkv, s.H, 2 * s.I})});
+}
+
+// The layer projections of M rows whose partial sums go to part floats.
+struct Projections { ProjPlan qkv, o, gate_up, down; };
+
+Projections plan_layer(const Shapes& s, long long M, size_t part) {
+    const int cus = device_cu_count();
+    auto plan = [&](int N, int K) {
+        return plan_proj((int)M, N, K, false, cus, (int)std::min<size_t>(part / ((size_t)M * N), 1024));
+    };
+    return {plan(s.Nqkv, s.H), plan(s.H, s.Nq), plan_proj((int)M, s.I, s.H, true, cus, 1), plan(s.H, s.I)};
+}
+
+// The same where they run beside the other half-batch's attention: splits of
+// at least 8 k-steps, 4 for the o and down projections (16 column blocks at
+// 1024 columns: 256 workgroups instead of 128).  Measured on a 28-layer B = 64
+// step: 20.79 ms against 20.98 ms with 2-step splits everywhere (the partials'
+// traffic outweighed the extra workgroups); o/down at 4 / 8 / 16 steps 20.76 /
+// 20.78 / 21.00 ms.
+struct BesideProjections { Gemm qkv, o, gate_up, down; };
+
+BesideProjections plan_beside(const Shapes& s, long long M, size_t part) {
+    const int cus = device_cu_count();
+    auto plan = [&](int N, int K, int min_steps) {
+        return Gemm{N, K, pick_split(N, K, cus, min_steps, part / (size_t)M)};
+    };
+    return {plan(s.Nqkv, s.H, 8), plan(s.H, s.Nq, 4), plan(2 * s.I, s.H, 8), plan(s.H, s.I, 4)};
 }
 
 template <class T>
@@ -542,12 +523,12 @@ sa_status grow(void** p, size_t* have, size_t need) {
 }
 
 // Logits of M rows and their greedy tokens: few rows take the streaming head
-// (in may hold the final norm's residual sum), more the tiled GEMM on in.x.
+// (in may hold the final norm's residual sum), more the tiled projection on in.x.
 sa_status head(sa_qwen3* m, const Shapes& s, const FewInput& in, int M, float* logits, int32_t* next,
                hipStream_t st) {
     if (few_rows_fit(M, s.H))
         return few_head(in, M, s.H, m->lm_head, s.V, logits, m->am_val, m->am_idx, next, st);
-    SA_TRY(gemm(in.x, M, m->lm_head, s.lm, logits, st));
+    SA_TRY(project(in.x, M, m->lm_head, plan_proj(M, s.V, s.H, false, device_cu_count(), 1), logits, st));
     hipLaunchKernelGGL(argmax_partial_kernel, dim3(kArgBlocks, M), dim3(256), 0, st, logits, s.V, m->am_val,
                        m->am_idx);
     SA_CHECK_LAUNCH();
@@ -602,7 +583,7 @@ extern "C" sa_status sa_qwen3_create(const sa_qwen3_desc* desc, int max_batch, s
         return s;
     };
     if (hipGetDevice(&m->device) != hipSuccess) return cleanup(fail(SA_EHIP, "hipGetDevice failed"));
-    const Shapes s = shapes_of(d, device_cu_count());
+    const Shapes s = shapes_of(d);
     const size_t H = s.H, V = s.V, B = max_batch;
     sa_status st;
     if ((st = dev_alloc(m, &m->embed, V * H)) != SA_OK) return cleanup(st);
@@ -656,7 +637,7 @@ extern "C" sa_status sa_qwen3_tensor_ptr(sa_qwen3* m, int layer, sa_qwen3_tensor
                                          sa_dtype* dtype) {
     clear_error();
     if (!m || !ptr || !count || !dtype) return fail(SA_EINVAL, "null argument");
-    const Shapes s = shapes_of(m->d, 1);
+    const Shapes s = shapes_of(m->d);
     const size_t H = s.H;
     const bool global = which == SA_QW_EMBED || which == SA_QW_FINAL_NORM || which == SA_QW_LM_HEAD;
     if (!global && (layer < 0 || layer >= m->d.num_layers)) return fail(SA_ERANGE, "layer out of range");
@@ -733,21 +714,13 @@ extern "C" sa_status sa_qwen3_prefill(sa_qwen3* m, sa_kvcache* cache, const int3
         if (sa_kvcache_capacity(cache, i) < L) return fail(SA_EFULL, "KV cache full, reserve pages for the prompt");
     }
     hipStream_t st = as_stream(stream);
-    const Shapes s = shapes_of(d, device_cu_count());
+    const Shapes s = shapes_of(d);
     const long long M = (long long)batch * L;
     if (M > 0x7fffffffLL / std::max({s.Nqkv, 2 * s.I, s.H}))
         return fail(SA_ERANGE, "batch * prompt too large");
     // K splits while the partial sums fit the widest projection's outputs.
-    const int cus = device_cu_count();
     const long long part_cols = std::max({s.Nqkv, 2 * s.I, s.H});
-    const int m_rows = (int)std::min<long long>(M, 0x7fffffff);
-    auto plan = [&](int N, int K, bool pair) {
-        return plan_proj(m_rows, N, K, pair, cus, (int)(part_cols / N));
-    };
-    const ProjPlan g_qkv = plan(s.Nqkv, s.H, false);
-    const ProjPlan g_o = plan(s.H, s.Nq, false);
-    const ProjPlan g_gu = plan(s.I, s.H, true);
-    const ProjPlan g_down = plan(s.H, s.I, false);
+    const Projections g = plan_layer(s, M, (size_t)M * part_cols);
 
     // activations of the M token rows, carved from one grow-only buffer
     const size_t f_x = M * s.H, f_q = M * s.Nq, f_k = M * s.Nk, f_act = M * s.I;
@@ -787,23 +760,23 @@ extern "C" sa_status sa_qwen3_prefill(sa_qwen3* m, sa_kvcache* cache, const int3
     for (int l = 0; l < d.num_layers; ++l) {
         const sa_qwen3::Layer& Ly = m->layers[l];
         // ---- attention block ----
-        SA_TRY(project(h, (int)M, Ly.qkv, g_qkv, part, st));
+        SA_TRY(project(h, (int)M, Ly.qkv, g.qkv, part, st));
         // q, k, v summed from the projection's split-K partials, q and k
         // normed and rotated (positions 0 .. L-1: the cache is empty), K and V
         // appended to the cache, q, k, v written for the attention: one launch.
-        SA_TRY(qknorm_rope_append_partials(cache, l, part, g_qkv.split, batch, L, s.Hq, Ly.q_norm, Ly.k_norm, eps,
+        SA_TRY(qknorm_rope_append_partials(cache, l, part, g.qkv.split, batch, L, s.Hq, Ly.q_norm, Ly.k_norm, eps,
                                            m->rope_cos, m->rope_sin, d.max_pos, q, k, v, st));
         SA_TRY(sa_prefill_causal_strided_ws(q, k, v, SA_DTYPE_F32, batch, s.Hq, s.Hkv, L, s.D, q_str, kv_str, q_str,
                                             scale, attn, attn_ws, ws_attn, stream));
-        SA_TRY(project(attn, (int)M, Ly.o, g_o, part, st));
-        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g_o.split, (int)M, s.H, x,
+        SA_TRY(project(attn, (int)M, Ly.o, g.o, part, st));
+        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g.o.split, (int)M, s.H, x,
                            Ly.post_norm, eps, h);
         SA_CHECK_LAUNCH();
         // ---- MLP ----
-        SA_TRY(project(h, (int)M, Ly.gate_up, g_gu, act, st));
-        SA_TRY(project(act, (int)M, Ly.down, g_down, part, st));
+        SA_TRY(project(h, (int)M, Ly.gate_up, g.gate_up, act, st));
+        SA_TRY(project(act, (int)M, Ly.down, g.down, part, st));
         const float* next_norm = l + 1 < d.num_layers ? m->layers[l + 1].in_norm : m->final_norm;
-        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g_down.split, (int)M, s.H,
+        hipLaunchKernelGGL(residual_norm_kernel, dim3((unsigned)M), dim3(256), 0, st, part, g.down.split, (int)M, s.H,
                            x, next_norm, eps, h);
         SA_CHECK_LAUNCH();
     }
@@ -834,7 +807,7 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     hipStream_t st = as_stream(stream);
     const size_t need = sa_paged_decode_ws_bytes(cache, batch, d.n_q_heads);
     SA_TRY(grow(&m->ws, &m->ws_bytes, need));
-    const Shapes s = shapes_of(d, device_cu_count());
+    const Shapes s = shapes_of(d);
     const int M = batch;
     const float eps = d.rms_eps;
     const float scale = 1.0f / sqrtf((float)d.head_dim);
@@ -854,18 +827,24 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         std::vector<int32_t> ids;
         bool few;
         float *x, *x_other, *o_part, *down_part;
+        bool beside;           // more rows: runs beside another half-batch's attention
+        Projections g;
+        BesideProjections gb;
     };
-    auto make_rows = [&](int r0, int n, float* part, void* ws, size_t ws_bytes, hipStream_t on) {
+    const size_t part_n = part_floats(s, m->max_batch);
+    auto make_rows = [&](int r0, int n, float* part, void* ws, size_t ws_bytes, hipStream_t on, bool beside) {
         float* o_part = part + (size_t)n * s.Nqkv;
         Rows r{r0, n, part, ws, ws_bytes, on, {}, few_rows_fit(n, s.H), m->x + (size_t)r0 * s.H,
-               m->x2 + (size_t)r0 * s.H, o_part, o_part + (size_t)kFewSplit * n * s.H};
+               m->x2 + (size_t)r0 * s.H, o_part, o_part + (size_t)kFewSplit * n * s.H,
+               beside, plan_layer(s, n, part_n), plan_beside(s, n, part_n)};
         for (int i = 0; i < n; ++i) r.ids.push_back(r0 + i);
         return r;
     };
-    const int ew_grid_full = std::min(4 * device_cu_count(), (M * s.I / 4 + 255) / 256);
     auto qkv = [&](Rows& r, int l) -> sa_status {
         const sa_qwen3::Layer& L = m->layers[l];
-        if (!r.few) return gemm(m->h + (size_t)r.r0 * s.H, r.n, L.qkv, s.qkv, r.part, r.st);
+        const float* h = m->h + (size_t)r.r0 * s.H;
+        if (!r.few && r.beside) return gemm(h, r.n, L.qkv, r.gb.qkv, r.part, r.st);
+        if (!r.few) return project(h, r.n, L.qkv, r.g.qkv, r.part, r.st);
         FewInput in{r.x, r.down_part, l ? kFewSplit : 0, L.in_norm, eps, l ? r.x_other : nullptr};
         SA_TRY(few_project_norm(in, r.n, s.H, L.qkv, s.Nqkv, r.part, r.st));
         if (l) std::swap(r.x, r.x_other);
@@ -877,7 +856,7 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     // (A separate split kernel cost 4.7 us per layer.)
     auto attention = [&](const Rows& r, int l) {
         const sa_qwen3::Layer& L = m->layers[l];
-        return sa::append_decode_partials(cache, l, r.part, r.few ? 1 : s.qkv.S, r.n, r.ids.data(), s.Hq, L.q_norm,
+        return sa::append_decode_partials(cache, l, r.part, r.few ? 1 : r.beside ? r.gb.qkv.S : r.g.qkv.split, r.n, r.ids.data(), s.Hq, L.q_norm,
                                           L.k_norm, eps, m->rope_cos, m->rope_sin, d.max_pos, scale,
                                           m->attn + (size_t)r.r0 * s.Nq, nullptr, r.ws, r.ws_bytes,
                                           l + 1 == d.num_layers ? 1 : 0, r.st);
@@ -903,18 +882,27 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
             SA_CHECK_LAUNCH();
             return SA_OK;
         }
-        SA_TRY(gemm(attn, r.n, L.o, s.o, r.part, r.st));
-        hipLaunchKernelGGL(residual_norm_kernel, dim3(r.n), dim3(256), 0, r.st, r.part, s.o.S, r.n, s.H, x,
-                           L.post_norm, eps, h);
-        SA_CHECK_LAUNCH();
-        SA_TRY(gemm(h, r.n, L.gate_up, s.gate_up, r.part, r.st));
-        const int ew_grid = std::min(ew_grid_full, (r.n * s.I / 4 + 255) / 256);
-        hipLaunchKernelGGL(swiglu_kernel, dim3(ew_grid), dim3(256), 0, r.st, r.part, s.gate_up.S, r.n, s.I, act);
-        SA_CHECK_LAUNCH();
-        SA_TRY(gemm(act, r.n, L.down, s.down, r.part, r.st));
-        hipLaunchKernelGGL(residual_norm_kernel, dim3(r.n), dim3(256), 0, r.st, r.part, s.down.S, r.n, s.H, x,
-                           next_norm, eps, h);
-        SA_CHECK_LAUNCH();
+        auto residual = [&](int split, const float* norm) -> sa_status {
+            hipLaunchKernelGGL(residual_norm_kernel, dim3(r.n), dim3(256), 0, r.st, r.part, split, r.n, s.H, x, norm,
+                               eps, h);
+            SA_CHECK_LAUNCH();
+            return SA_OK;
+        };
+        if (r.beside) {
+            SA_TRY(gemm(attn, r.n, L.o, r.gb.o, r.part, r.st));
+            SA_TRY(residual(r.gb.o.S, L.post_norm));
+            SA_TRY(gemm(h, r.n, L.gate_up, r.gb.gate_up, r.part, r.st));
+            const int grid = std::min(4 * device_cu_count(), (r.n * s.I / 4 + 255) / 256);
+            hipLaunchKernelGGL(swiglu_kernel, dim3(grid), dim3(256), 0, r.st, r.part, r.gb.gate_up.S, r.n, s.I, act);
+            SA_CHECK_LAUNCH();
+            SA_TRY(gemm(act, r.n, L.down, r.gb.down, r.part, r.st));
+            return residual(r.gb.down.S, next_norm);
+        }
+        SA_TRY(project(attn, r.n, L.o, r.g.o, r.part, r.st));
+        SA_TRY(residual(r.g.o.split, L.post_norm));
+        SA_TRY(project(h, r.n, L.gate_up, r.g.gate_up, act, r.st));
+        SA_TRY(project(act, r.n, L.down, r.g.down, r.part, r.st));
+        SA_TRY(residual(r.g.down.split, next_norm));
         return SA_OK;
     };
 
@@ -941,7 +929,7 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     const long long attn_bytes = total * d.n_kv_heads * d.head_dim * 2LL * kv_elem;
     const char* fenv = std::getenv("SA_DECODE_INTERLEAVE");
     const bool interleave = M >= 2 && (fenv ? std::atoi(fenv) != 0 : attn_bytes >= kInterleaveBytes);
-    Rows all = make_rows(0, M, m->part, m->ws, m->ws_bytes, st);
+    Rows all = make_rows(0, M, m->part, m->ws, m->ws_bytes, st, false);
     few_head_rows = all.few && !interleave;
     if (!interleave) {
         for (int l = 0; l < d.num_layers; ++l) {
@@ -954,8 +942,8 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         SA_TRY(grow(&m->ws2, &m->ws2_bytes, need));
         int cut = 1;
         while (cut < M - 1 && 2 * prefix[cut] < total) ++cut;
-        Rows a = make_rows(0, cut, m->part, m->ws, m->ws_bytes, st);
-        Rows b = make_rows(cut, M - cut, m->part2, m->ws2, m->ws2_bytes, m->side);
+        Rows a = make_rows(0, cut, m->part, m->ws, m->ws_bytes, st, true);
+        Rows b = make_rows(cut, M - cut, m->part2, m->ws2, m->ws2_bytes, m->side, true);
         hipEvent_t fork = m->events[0], join = m->events[1], a_first = m->events[2];
         SA_HIP_TRY(hipEventRecord(fork, st));
         SA_HIP_TRY(hipStreamWaitEvent(m->side, fork, 0));
