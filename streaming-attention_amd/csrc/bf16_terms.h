@@ -1,6 +1,7 @@
 // fp32 activations as bf16 MFMA operands: three bf16 terms per value.
 #pragma once
 
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace sa {

@@ -103,6 +103,7 @@ struct DecodeArgs {
     // hold tokens, sequence i's at cstart[i] .. cstart[i + 1] - 1 (entries
     // past the launch's sequences hold INT_MAX), and blockIdx.z is 0.
     int compact;
+    int leave_parts;         // host: no merge launch, the consumer merges
     // Paged, not FUSED: the committed lengths come from pos (host values)
     // instead of seq_lens.
     int host_lens;
@@ -816,7 +817,7 @@ sa_status launch_decode(const DecodeArgs& a, int n_seq, hipStream_t st) {
         hipLaunchKernelGGL((split_kv_decode_kernel<D, NREP, BF16, PAGED, W, FUSED>), grid, dim3(W * kWave), 0, st, a);
     }
     SA_CHECK_LAUNCH();
-    if (a.n_split > 1) {
+    if (a.n_split > 1 && !a.leave_parts) {
         const dim3 mgrid(n_seq * a.n_q);
         // Rows with many chunks: four 256-thread workgroups per row, each
         // merging a quarter of head_dim (their block reductions span 4
@@ -1006,6 +1007,12 @@ sa_status decode_paged_fused(const PagedView& c, const float* q, int n_seq, cons
     if (need > 0) {
         if (!ws || ws_bytes < need) return fail(SA_ENOMEM, "workspace too small for split-KV partials");
         carve_ws(a, ws, bh);
+    }
+    if (f.parts) {
+        a.leave_parts = a.n_split <= parts_limit(n_seq);
+        *f.parts = {a.part_ml, a.part_o, a.leave_parts && a.n_split > 1 ? a.n_split : 0, {}};
+        for (int i = 0; a.leave_parts && i < n_seq; ++i)
+            f.parts->n_act[i] = (std::min(f.pos[i] + 1, c.max_pages * 64) + a.chunk - 1) / a.chunk;
     }
     for (int i0 = 0; i0 < n_seq; i0 += kRowsPerLaunch) {
         const int m = std::min(kRowsPerLaunch, n_seq - i0);

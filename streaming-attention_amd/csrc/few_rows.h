@@ -29,8 +29,11 @@ bool few_rows_fit(int rows, int hidden);
 sa_status few_project_norm(const FewInput& in, int M, int K, const uint16_t* W, int N, float* out, hipStream_t st);
 // out[M][I] = silu(gate) * up of input . W^T, W [2 I][K] (gate rows, then up).
 sa_status few_gate_up(const FewInput& in, int M, int K, const uint16_t* W, int I, float* out, hipStream_t st);
-// out[kFewSplit][M][N]: the K splits of x . W^T.
-sa_status few_project_split(const float* x, int M, int K, const uint16_t* W, int N, float* out, hipStream_t st);
+// out[kFewSplit][M][N]: the K splits of x . W^T.  With parts (n_split > 0) rows of
+// several partials are merged from them instead of read from x: K = heads of
+// D columns (D a multiple of 4), at most parts_limit(M) partials.
+sa_status few_project_split(const float* x, int M, int K, const uint16_t* W, int N, float* out, hipStream_t st,
+                            const DecodeParts* parts = nullptr, int D = 0);
 // logits[M][N] = input . W^T and next[m] = the lowest index of row m's maximum;
 // am_val / am_idx: [M][kFewHeadBlocks] scratch.
 sa_status few_head(const FewInput& in, int M, int K, const uint16_t* W, int N, float* logits, float* am_val,

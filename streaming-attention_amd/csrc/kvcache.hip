@@ -680,7 +680,8 @@ sa_status append_decode_impl(sa_kvcache* c, int layer, const float* q, const flo
                              const float* part, int n_part, int n_seq, const int32_t* seq_ids, int n_q_heads,
                              const float* q_norm_w, const float* k_norm_w, float eps, const float* rope_cos,
                              const float* rope_sin, int rope_max_pos, float scale, float* out, float* q_out,
-                             void* ws, size_t ws_bytes, int commit, hipStream_t stream) {
+                             void* ws, size_t ws_bytes, int commit, hipStream_t stream,
+                             DecodeParts* parts = nullptr) {
     if (!valid_cache(c)) return fail(SA_EINVAL, "invalid cache");
     if (layer < 0 || layer >= c->desc.num_layers) return fail(SA_ERANGE, "Layer index out of range");
     if (!out || (part ? n_part <= 0 : (!q || !k || !v))) return fail(SA_EINVAL, "null q, k, v or out");
@@ -713,6 +714,7 @@ sa_status append_decode_impl(sa_kvcache* c, int layer, const float* q, const flo
     const bool in_kernel_commit = commit && n_seq <= kRowsPerLaunch;
     f.q_out = q_out; f.lens = c->d_lens; f.pos = pos.data(); f.commit = in_kernel_commit;
     f.part = part; f.part_S = n_part; f.part_M = n_seq;
+    f.parts = parts;
     SA_TRY(decode_paged_fused(pv, q, n_seq, seq_ids, n_q_heads, f, max_len, total, scale, out, ws, ws_bytes,
                               stream));
     if (commit) {
@@ -729,11 +731,11 @@ sa_status append_decode_partials(sa_kvcache* c, int layer, const float* part, in
                                  const int32_t* seq_ids, int n_q_heads, const float* q_norm_w,
                                  const float* k_norm_w, float eps, const float* rope_cos, const float* rope_sin,
                                  int rope_max_pos, float scale, float* out, float* q_out, void* ws,
-                                 size_t ws_bytes, int commit, hipStream_t st) {
+                                 size_t ws_bytes, int commit, hipStream_t st, DecodeParts* parts) {
     if (!part) return fail(SA_EINVAL, "null projection partials");
     return append_decode_impl(c, layer, nullptr, nullptr, nullptr, part, n_part, n_seq, seq_ids, n_q_heads,
                               q_norm_w, k_norm_w, eps, rope_cos, rope_sin, rope_max_pos, scale, out, q_out, ws,
-                              ws_bytes, commit, st);
+                              ws_bytes, commit, st, parts);
 }
 
 }  // namespace sa

@@ -830,13 +830,14 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         bool beside;           // more rows: runs beside another half-batch's attention
         Projections g;
         BesideProjections gb;
+        DecodeParts parts;     // few rows: the attention's unmerged partials
     };
     const size_t part_n = part_floats(s, m->max_batch);
     auto make_rows = [&](int r0, int n, float* part, void* ws, size_t ws_bytes, hipStream_t on, bool beside) {
         float* o_part = part + (size_t)n * s.Nqkv;
         Rows r{r0, n, part, ws, ws_bytes, on, {}, few_rows_fit(n, s.H), m->x + (size_t)r0 * s.H,
                m->x2 + (size_t)r0 * s.H, o_part, o_part + (size_t)kFewSplit * n * s.H,
-               beside, plan_layer(s, n, part_n), plan_beside(s, n, part_n)};
+               beside, plan_layer(s, n, part_n), plan_beside(s, n, part_n), {}};
         for (int i = 0; i < n; ++i) r.ids.push_back(r0 + i);
         return r;
     };
@@ -854,12 +855,12 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     // the paged decode in one launch per 64 sequences (plus the LSE merge of
     // multi-chunk sequences); the last layer's call also commits the token.
     // (A separate split kernel cost 4.7 us per layer.)
-    auto attention = [&](const Rows& r, int l) {
+    auto attention = [&](Rows& r, int l) {
         const sa_qwen3::Layer& L = m->layers[l];
         return sa::append_decode_partials(cache, l, r.part, r.few ? 1 : r.beside ? r.gb.qkv.S : r.g.qkv.split, r.n, r.ids.data(), s.Hq, L.q_norm,
                                           L.k_norm, eps, m->rope_cos, m->rope_sin, d.max_pos, scale,
                                           m->attn + (size_t)r.r0 * s.Nq, nullptr, r.ws, r.ws_bytes,
-                                          l + 1 == d.num_layers ? 1 : 0, r.st);
+                                          l + 1 == d.num_layers ? 1 : 0, r.st, r.few ? &r.parts : nullptr);
     };
     // o projection, residual + norm, MLP, residual + the next block's norm
     // (few rows: the last two are left to the launch that reads the sum).
@@ -871,7 +872,7 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         float* act = m->act + (size_t)r.r0 * s.I;
         const float* next_norm = l + 1 < d.num_layers ? m->layers[l + 1].in_norm : m->final_norm;
         if (r.few) {
-            SA_TRY(few_project_split(attn, r.n, s.Nq, L.o, s.H, r.o_part, r.st));
+            SA_TRY(few_project_split(attn, r.n, s.Nq, L.o, s.H, r.o_part, r.st, &r.parts, s.D));
             FewInput in{r.x, r.o_part, kFewSplit, L.post_norm, eps, r.x_other};
             SA_TRY(few_gate_up(in, r.n, s.H, L.gate_up, s.I, act, r.st));
             std::swap(r.x, r.x_other);

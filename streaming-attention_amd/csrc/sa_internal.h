@@ -261,12 +261,28 @@ sa_status qknorm_rope_append_partials(sa_kvcache* c, int layer, const float* par
                                       const float* rope_cos, const float* rope_sin, int rope_max_pos, float* q_out,
                                       float* k_out, float* v_out, hipStream_t st);
 
+// The split-KV partials of a decode launch whose consumer merges them: row m's
+// query head h has n_act[m] of them (one or none: its output was written as
+// usual), partial i's (m, l) at ml[((m n_q + h) n_split + i) 2] and its D floats
+// O, relative to that m, at o[((m n_q + h) n_split + i) D].
+constexpr int kPartsRows = 8, kPartsMax = 8;
+// The most partials per row that M rows' consumer holds in registers.
+inline int parts_limit(int M) { return M <= 2 ? 8 : M <= 4 ? 4 : M <= kPartsRows ? 2 : 1; }
+struct DecodeParts {
+    const float* ml;
+    const float* o;
+    int n_split;             // 0: nothing to merge
+    int n_act[kPartsRows];
+};
+
 // sa_append_decode with q, k and v read from split-K partials (FusedAppend).
+// parts, if given: a launch of at most parts_limit chunks per sequence leaves
+// its partials for the caller to merge (n_split > 1).
 sa_status append_decode_partials(sa_kvcache* c, int layer, const float* part, int n_part, int n_seq,
                                  const int32_t* seq_ids, int n_q_heads, const float* q_norm_w,
                                  const float* k_norm_w, float eps, const float* rope_cos, const float* rope_sin,
                                  int rope_max_pos, float scale, float* out, float* q_out, void* ws,
-                                 size_t ws_bytes, int commit, hipStream_t st);
+                                 size_t ws_bytes, int commit, hipStream_t st, DecodeParts* parts = nullptr);
 
 size_t paged_ws(int n_seq, int n_q, int n_kv, int d, int max_pages);
 // seq_ids: host array of cache rows (NULL: 0 .. n_seq-1), already checked.
@@ -301,6 +317,7 @@ struct FusedAppend {
     const float* part = nullptr;
     int part_S = 0;
     int part_M = 0;
+    DecodeParts* parts = nullptr;   // see append_decode_partials
 };
 
 // decode_paged with the step's append folded in: one launch per
