@@ -34,6 +34,8 @@ sa_status few_gate_up(const FewInput& in, int M, int K, const uint16_t* W, int I
 // D columns (D a multiple of 4), at most parts_limit(M) partials.
 sa_status few_project_split(const float* x, int M, int K, const uint16_t* W, int N, float* out, hipStream_t st,
                             const DecodeParts* parts = nullptr, int D = 0);
+// next[m] = the greedy index of row m's nb workgroup maxima pv / pi [M][nb].
+sa_status few_argmax(const float* pv, const int32_t* pi, int nb, int M, int32_t* next, hipStream_t st);
 // logits[M][N] = input . W^T and next[m] = the lowest index of row m's maximum;
 // am_val / am_idx: [M][kFewHeadBlocks] scratch.
 sa_status few_head(const FewInput& in, int M, int K, const uint16_t* W, int N, float* logits, float* am_val,

@@ -450,7 +450,11 @@ sa_status few_head(const FewInput& in, int M, int K, const uint16_t* W, int N, f
     hipLaunchKernelGGL(few_head_kernel, dim3(kFewHeadBlocks), dim3(kHeadWaves * 64), bytes, st,
                        HeadArgs{in, W, logits, am_val, am_idx, M, K, N});
     SA_CHECK_LAUNCH();
-    hipLaunchKernelGGL(few_argmax_kernel, dim3(M), dim3(64), 0, st, am_val, am_idx, kFewHeadBlocks, next);
+    return few_argmax(am_val, am_idx, kFewHeadBlocks, M, next, st);
+}
+
+sa_status few_argmax(const float* pv, const int32_t* pi, int nb, int M, int32_t* next, hipStream_t st) {
+    hipLaunchKernelGGL(few_argmax_kernel, dim3(M), dim3(64), 0, st, pv, pi, nb, next);
     SA_CHECK_LAUNCH();
     return SA_OK;
 }
