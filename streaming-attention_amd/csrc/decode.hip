@@ -1001,6 +1001,14 @@ sa_status decode_paged_fused(const PagedView& c, const float* q, int n_seq, cons
     // The same chunking as decode_paged with one pending token.
     a.chunk = pick_chunk(total_len * c.n_kv, (long long)c.max_pages * 64, (long long)kMaxChunkPages * 64);
     if (a.chunk > kMaxChunkPages * 64) return fail(SA_EINVAL, "max_pages_per_seq too large for the split cap");
+    // Partials that the consumer merges cost no launch: the smallest chunks, one
+    // tile per wave, while it takes that many and they are one round of
+    // workgroups.  28 layers, one sequence of 513 - 613 tokens: 11.0 ->
+    // 8.6 us of attention per layer, 1010 -> 975 us per step.
+    const int small = (max_len + kMinChunk - 1) / kMinChunk;
+    if (f.parts && forced_chunk() <= 0 && a.chunk > kMinChunk && small <= parts_limit(n_seq) &&
+        (long long)small * c.n_kv * n_seq <= device_cu_count())
+        a.chunk = kMinChunk;
     a.n_split = (max_len + a.chunk - 1) / a.chunk;
     const long long bh = (long long)std::min(n_seq, kRowsPerLaunch) * n_q;
     const size_t need = ws_bytes_for(bh, a.n_split, c.d);

@@ -31,7 +31,7 @@ sa_status few_project_norm(const FewInput& in, int M, int K, const uint16_t* W, 
 sa_status few_gate_up(const FewInput& in, int M, int K, const uint16_t* W, int I, float* out, hipStream_t st);
 // out[kFewSplit][M][N]: the K splits of x . W^T.  With parts (n_split > 0) rows of
 // several partials are merged from them instead of read from x: K = heads of
-// D columns (D a multiple of 4), at most parts_limit(M) partials.
+// D columns (D a power of two, 4 or more), at most parts_limit(M) partials.
 sa_status few_project_split(const float* x, int M, int K, const uint16_t* W, int N, float* out, hipStream_t st,
                             const DecodeParts* parts = nullptr, int D = 0);
 // next[m] = the greedy index of row m's nb workgroup maxima pv / pi [M][nb].

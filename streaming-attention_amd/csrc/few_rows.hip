@@ -35,8 +35,8 @@ struct FewArgs {
     const uint16_t* w;   // [N or 2 N][K]
     float* out;          // [split][M][N]
     int M, K, N;
-    DecodeParts parts;   // NS > 0
-    int D;
+    DecodeParts parts;   // NS > 0: partials of heads of 1 << d_log2 columns
+    int d_log2;
 };
 
 // Workgroup (bx, by) owns 16 output columns (kSwiglu: 16 gate and the 16 up
@@ -58,7 +58,8 @@ struct FewArgs {
 // NS > 0: the rows are attention outputs left as up to NS split-KV partials,
 // merged here; their (m, l) and O are all loaded before the first use, in the
 // round trip that would load the merged rows.  The merge launch this saves
-// took 4.0 us of a layer, these loads add 0.5 to the projection's 4.6.
+// took 4.0 us of a layer; these loads add 0.5 (3 partials) to 2.3 (5, the
+// 8-partial form) to the projection's 4.4.
 template <int W, int RP, int PRO, int EPI, int NS = 0>
 __global__ void __launch_bounds__(W * 64)
 few_rows_kernel(FewArgs a) {
@@ -117,21 +118,21 @@ few_rows_kernel(FewArgs a) {
 #pragma unroll
         for (int i = 0; i < RP; ++i) at[i] = (size_t)min(2 * i + half, M - 1) * K + k;
         if constexpr (NS > 0) {
-            const int head = (int)k / a.D, d = (int)k - head * a.D;
+            const int D = 1 << a.d_log2, head = (int)k >> a.d_log2, d = (int)k & (D - 1);
 #pragma unroll
             for (int i = 0; i < RP; ++i) {
                 const int m = min(2 * i + half, M - 1), n = a.parts.n_act[m];
-                const size_t p0 = ((size_t)m * (K / a.D) + head) * a.parts.n_split;
+                const int p0 = (m * (K >> a.d_log2) + head) * a.parts.n_split;
                 // One partial or none: the row itself, with weight 1.
-                const float* o = n > 1 ? a.parts.o + p0 * a.D + d : a.in.x + at[i];
-                const float* ml = a.parts.ml + 2 * p0;
+                const float* o = n > 1 ? a.parts.o + ((size_t)p0 << a.d_log2) + d : a.in.x + at[i];
+                const float2* ml = reinterpret_cast<const float2*>(a.parts.ml) + p0;
                 f32x4_t y[NS];
                 float2 w[NS];
 #pragma unroll
                 for (int s = 0; s < NS; ++s) {
-                    const int c = max(min(s, n - 1), 0);
-                    w[s] = *reinterpret_cast<const float2*>(ml + 2 * (n > 1 ? c : 0));
-                    y[s] = *reinterpret_cast<const f32x4_t*>(o + (size_t)c * a.D);
+                    const int c = s < n ? s : 0;
+                    w[s] = ml[c];
+                    y[s] = *reinterpret_cast<const f32x4_t*>(o + (c << a.d_log2));
                 }
                 float mx = w[0].x;
 #pragma unroll
@@ -433,11 +434,12 @@ sa_status few_gate_up(const FewInput& in, int M, int K, const uint16_t* W, int I
 
 sa_status few_project_split(const float* x, int M, int K, const uint16_t* W, int N, float* out, hipStream_t st,
                             const DecodeParts* parts, int D) {
-    FewArgs a{{x, nullptr, 0, nullptr, 0.f, nullptr}, W, out, M, K, N, {}, D};
+    FewArgs a{{x, nullptr, 0, nullptr, 0.f, nullptr}, W, out, M, K, N, {}, 0};
     const dim3 grid(N / 16, kFewSplit);
     if (!parts || parts->n_split <= 1) return launch_rows<16, kPlain, kOut>(a, grid, st);
     if (parts->n_split > parts_limit(M)) return fail(SA_EINVAL, "more partials than the rows can merge");
     a.parts = *parts;
+    a.d_log2 = __builtin_ctz(D);
     if (parts->n_split <= 2) return launch_rows<16, kPlain, kOut, 2>(a, grid, st);
     if (parts->n_split <= 4) return launch_rows<16, kPlain, kOut, 4>(a, grid, st);
     return launch_rows<16, kPlain, kOut, kPartsMax>(a, grid, st);

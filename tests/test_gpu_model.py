@@ -288,3 +288,21 @@ def test_model_decode_few_rows(sa, oracle, synth, interleave, rows, hidden, inte
     lens = [1 + (37 * i) % 150 for i in range(rows)]
     run_parity(sa, oracle, synth, cfg, 0.05, lens, 3, sa.SA_DTYPE_F32, 60 + rows,
                [(11 * i + 3) % vocab for i in range(rows)], check)
+
+
+# Partials merged by the o projection: 2 .. 8 chunks of 128 tokens for up to
+# 2 rows, 4 for up to 4, 2 for up to 8, beside rows of one chunk; one chunk
+# more than the limit takes the merge launch.
+@pytest.mark.parametrize("lens", [[130], [1023], [1024], [30, 600], [257, 127, 510], [512, 5, 1, 300], [511, 513, 64, 9],
+                                  [255, 3, 200, 128, 127], [100, 129, 254, 17, 64, 250, 1, 255], [256] * 7])
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_model_decode_merged_partials(sa, oracle, synth, lens, head_dim):
+    """fp32 KV: as test_model_decode_fp32_kv, rows at the edges of the chunk
+    counts a few-row step's o projection merges."""
+    cfg = dict(SMALL, num_layers=1, head_dim=head_dim)
+
+    def check(t, got, want):
+        assert np.abs(got - want).max() <= 1e-4, t
+        assert rel_l2(got, want) <= 1e-5, t
+    run_parity(sa, oracle, synth, cfg, 0.1, lens, 2, sa.SA_DTYPE_F32, 31 + len(lens), [3 + b for b in range(len(lens))],
+               check)
