@@ -45,17 +45,20 @@ struct Tile {
 // KW parts are staged as bf16 terms (double-buffered, one barrier per stage);
 // the wave's weights go through LDS it has to itself, two steps at a time, so
 // that global loads cover whole 128-byte lines (an MFMA fragment loaded from
-// global memory, 16 rows per 16 lanes, takes 64 cycles of address processing
-// per KiB; a line-wise load 27).  PAIR: the first half of the column groups
-// computes gate columns, the second the up columns beside them, and SwiGLU is
-// applied where their sums meet.
+// global memory, 16 rows per 16 lanes, took 2.4 times as long per KiB).  PAIR:
+// the first half of the column groups computes gate columns, the second the up
+// columns beside them, and SwiGLU is applied where their sums meet.
 //
-// Bound: LDS.  Its port moves 64 bytes per cycle, so the 16 fragment reads of
-// a 64 x 64 wave step take 256 cycles per CU where its 48 MFMAs take 192, and
-// the staging writes add 128 to 160: a stage of 8 wave steps measures 1.10 to
-// 1.20 us against 0.64 us of MFMA.  64 x 64 per wave (32 x 64 for few rows) has
-// the fewest reads per MFMA that leave the registers two waves per SIMD; the
-// k parts let small grids keep it.  The split into terms runs between MFMAs.
+// 64 x 64 per wave (32 x 64 for few rows) has the fewest LDS reads per MFMA, 16
+// per 48, that leave the registers two waves per SIMD; the k parts let small
+// grids keep it.  The row reads run one block ahead of their MFMAs and the
+// split into terms runs between them.
+//
+// Bound: the serial course of a stage (weight store, first fragment reads,
+// MFMAs, barrier, all waves in step) and of a workgroup's start and end; no
+// unit is full.  Counters of the 4096 x 1024 launch at 512 rows, of 36,900 cycles per
+// CU: MFMA 12,300, LDS 10,750 without bank conflicts, VALU 11,700.  A stage of 8
+// wave steps measures 1.10 to 1.20 us against 0.64 us of MFMA.
 //
 // Measured (weights from HBM): 4096 x 1024 at 512 rows 17.2 us (64 x 64 tiles
 // of 4 waves with weight fragments from global memory: 23.2), 1024 x 2048 12.0
