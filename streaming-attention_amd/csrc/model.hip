@@ -448,7 +448,7 @@ Shapes shapes_of(const sa_qwen3_desc& d) {
     return s;
 }
 
-// Floats of the partial-sum buffer of a decode step of up to B rows: a
+// Floats of the partial-sum buffer of a decode step or prompt of up to B rows: a
 // few-row step's q | k | v and its o and down splits, or 8 splits of the wider of
 // qkv and o / down for up to 128 rows (more rows take fewer), gate and up unsplit.
 size_t part_floats(const Shapes& s, size_t B) {
@@ -714,13 +714,11 @@ extern "C" sa_status sa_qwen3_prefill(sa_qwen3* m, sa_kvcache* cache, const int3
     const long long M = (long long)batch * L;
     if (M > 0x7fffffffLL / std::max({s.Nqkv, 2 * s.I, s.H}))
         return fail(SA_ERANGE, "batch * prompt too large");
-    // K splits while the partial sums fit the widest projection's outputs.
-    const long long part_cols = std::max({s.Nqkv, 2 * s.I, s.H});
-    const Projections g = plan_layer(s, M, (size_t)M * part_cols);
+    const size_t f_part = part_floats(s, (size_t)M);
+    const Projections g = plan_layer(s, M, f_part);
 
     // activations of the M token rows, carved from one grow-only buffer
     const size_t f_x = M * s.H, f_q = M * s.Nq, f_k = M * s.Nk, f_act = M * s.I;
-    const size_t f_part = M * part_cols;
     // the attention's workspace (paired key ranges of short prompts) after
     // the activations, at a 256-byte boundary
     const size_t ws_attn = sa_prefill_causal_ws_bytes(SA_DTYPE_F32, batch, s.Hq, s.Hkv, L, s.D);
