@@ -58,8 +58,8 @@ struct FewArgs {
 // NS > 0: the rows are attention outputs left as up to NS split-KV partials,
 // merged here; their (m, l) and O are all loaded before the first use, in the
 // round trip that would load the merged rows.  The merge launch this saves
-// took 4.0 us of a layer; these loads add 0.5 (3 partials) to 2.3 (5, the
-// 8-partial form) to the projection's 4.4.
+// took 4.0 us of a layer; these loads add 0.5 (3 partials) to 1.6 (5; 2.3
+// in the 8-partial form) to the projection's 4.4.
 template <int W, int RP, int PRO, int EPI, int NS = 0>
 __global__ void __launch_bounds__(W * 64)
 few_rows_kernel(FewArgs a) {
@@ -442,6 +442,7 @@ sa_status few_project_split(const float* x, int M, int K, const uint16_t* W, int
     a.d_log2 = __builtin_ctz(D);
     if (parts->n_split <= 2) return launch_rows<16, kPlain, kOut, 2>(a, grid, st);
     if (parts->n_split <= 4) return launch_rows<16, kPlain, kOut, 4>(a, grid, st);
+    if (parts->n_split <= 6) return launch_rows<16, kPlain, kOut, 6>(a, grid, st);
     return launch_rows<16, kPlain, kOut, kPartsMax>(a, grid, st);
 }
 
