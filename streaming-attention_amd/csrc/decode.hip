@@ -1017,10 +1017,8 @@ sa_status decode_paged_fused(const PagedView& c, const float* q, int n_seq, cons
         carve_ws(a, ws, bh);
     }
     if (f.parts) {
-        a.leave_parts = a.n_split <= parts_limit(n_seq);
-        *f.parts = {a.part_ml, a.part_o, a.leave_parts && a.n_split > 1 ? a.n_split : 0, {}};
-        for (int i = 0; a.leave_parts && i < n_seq; ++i)
-            f.parts->n_act[i] = (std::min(f.pos[i] + 1, c.max_pages * 64) + a.chunk - 1) / a.chunk;
+        *f.parts = plan_parts(a.part_ml, a.part_o, n_seq, a.n_split, a.chunk, c.max_pages * 64, f.pos);
+        a.leave_parts = f.parts->n_split > 0;
     }
     for (int i0 = 0; i0 < n_seq; i0 += kRowsPerLaunch) {
         const int m = std::min(kRowsPerLaunch, n_seq - i0);

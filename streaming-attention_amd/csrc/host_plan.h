@@ -1,0 +1,38 @@
+// Host-only planning of launches (no HIP): plain integers, so that it is
+// tested without a GPU.
+#pragma once
+
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace sa {
+
+// The split-KV partials of a decode launch whose consumer merges them: row m's
+// query head h has n_act[m] of them (one or none: its output was written as
+// usual), partial i's (m, l) at ml[((m n_q + h) n_split + i) 2] and its D floats
+// O, relative to that m, at o[((m n_q + h) n_split + i) D].
+constexpr int kPartsRows = 8, kPartsMax = 8;
+struct DecodeParts {
+    const float* ml;
+    const float* o;
+    int n_split;             // 0: nothing to merge, n_act unset
+    int n_act[kPartsRows];
+};
+
+// The most partials per row that M rows' consumer holds in registers.
+inline int parts_limit(int M) { return M <= 2 ? 8 : M <= 4 ? 4 : M <= kPartsRows ? 2 : 1; }
+
+// The partials that a launch of n_seq rows in n_split chunks leaves to its
+// consumer: those of at most parts_limit chunks, so of at most kPartsRows rows.
+// Row i holds tokens 0 .. pos[i] of at most capacity.
+inline DecodeParts plan_parts(const float* ml, const float* o, int n_seq, int n_split, int chunk, int capacity,
+                              const int32_t* pos) {
+    DecodeParts p{ml, o, 0, {}};
+    if (n_split <= 1 || n_split > parts_limit(n_seq)) return p;
+    p.n_split = n_split;
+    for (int i = 0; i < n_seq; ++i) p.n_act[i] = (std::min(pos[i] + 1, capacity) + chunk - 1) / chunk;
+    return p;
+}
+
+}  // namespace sa

@@ -5,6 +5,7 @@
 #include <stdint.h>
 #include <string>
 
+#include "host_plan.h"
 #include "sa_amd.h"
 
 namespace sa {
@@ -260,20 +261,6 @@ sa_status qknorm_rope_append_partials(sa_kvcache* c, int layer, const float* par
                                       int n_q_heads, const float* q_norm_w, const float* k_norm_w, float eps,
                                       const float* rope_cos, const float* rope_sin, int rope_max_pos, float* q_out,
                                       float* k_out, float* v_out, hipStream_t st);
-
-// The split-KV partials of a decode launch whose consumer merges them: row m's
-// query head h has n_act[m] of them (one or none: its output was written as
-// usual), partial i's (m, l) at ml[((m n_q + h) n_split + i) 2] and its D floats
-// O, relative to that m, at o[((m n_q + h) n_split + i) D].
-constexpr int kPartsRows = 8, kPartsMax = 8;
-// The most partials per row that M rows' consumer holds in registers.
-inline int parts_limit(int M) { return M <= 2 ? 8 : M <= 4 ? 4 : M <= kPartsRows ? 2 : 1; }
-struct DecodeParts {
-    const float* ml;
-    const float* o;
-    int n_split;             // 0: nothing to merge
-    int n_act[kPartsRows];
-};
 
 // sa_append_decode with q, k and v read from split-K partials (FusedAppend).
 // parts, if given: a launch of at most parts_limit chunks per sequence leaves
