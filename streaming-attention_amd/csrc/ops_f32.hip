@@ -27,13 +27,20 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // 64 x 32 blocks of x and w through LDS, k-major, so that a fragment read
 // (lane l: row l & 15 at k = l >> 4) is 16 consecutive floats per k.  Rows,
 // columns and k past the matrix read as zero; stores are bounds-checked.
-// For K and pointers that float4 loads cannot take (K % 4 != 0, x or w not
-// 16-byte aligned); the others take linear_f32_direct_kernel.
+//
+// VEC: K % 4 == 0 and 16-byte aligned x and w, so blocks load as float4; such
+// calls take linear_f32_direct_kernel where launch_vec expects it to be faster.
+// Here every step's 32 products per output are added up by themselves and then
+// added to the sum, so no chain is longer than that kernel's: 1.5e-7 of the
+// result in the 2-norm at K = 1024 (2.9e-7 there, 5.7e-7 in one chain over K).
+// Eight workgroups share a CU and hide each other's staging; with the registers
+// for five, 1024 rows times 6144 x 1024 take 174 us instead of 147.
 // ---------------------------------------------------------------------------
 constexpr int kLinTile = 64;
 constexpr int kLinK = 32;
 constexpr int kLinStride = kLinTile + 4;   // floats per LDS k row
 
+template <bool VEC>
 __device__ __forceinline__ void stage_block(const float* __restrict__ src, int rows, int K, int r0, int k0,
                                             float (*dst)[kLinStride]) {
 #pragma unroll
@@ -44,16 +51,21 @@ __device__ __forceinline__ void stage_block(const float* __restrict__ src, int r
         f32x4_t v = {0.f, 0.f, 0.f, 0.f};
         if (row < rows) {
             const float* p = src + (size_t)row * K + k;
+            if constexpr (VEC) {
+                if (k < K) v = *reinterpret_cast<const f32x4_t*>(p);
+            } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (k + j < K) v[j] = p[j];
+                for (int j = 0; j < 4; ++j)
+                    if (k + j < K) v[j] = p[j];
+            }
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) dst[kq + j][r] = v[j];
     }
 }
 
-__global__ void __launch_bounds__(256)
+template <bool VEC>
+__global__ void __launch_bounds__(256, VEC ? 8 : 1)
 linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
                   float* __restrict__ y, int M, int N, int K) {
     __shared__ float xs[kLinK][kLinStride];
@@ -62,15 +74,10 @@ linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, cons
     const int m0 = blockIdx.y * kLinTile, n0 = blockIdx.x * kLinTile;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     const int c = lane & 15, kl = lane >> 4;
-    f32x4_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
+    f32x4_t sum[2][2] = {}, acc[2][2] = {};
     for (int k0 = 0; k0 < K; k0 += kLinK) {
-        stage_block(x, M, K, m0, k0, xs);
-        stage_block(w, N, K, n0, k0, ws);
+        stage_block<VEC>(x, M, K, m0, k0, xs);
+        stage_block<VEC>(w, N, K, n0, k0, ws);
         __syncthreads();
 #pragma unroll
         for (int ks = 0; ks < kLinK; ks += 4) {
@@ -81,6 +88,15 @@ linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, cons
             acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, acc[0][1], 0, 0, 0);
             acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, acc[1][0], 0, 0, 0);
             acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc[1][1], 0, 0, 0);
+        }
+        if constexpr (VEC) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = f32x4_t{};
+                }
         }
         __syncthreads();
     }
@@ -95,7 +111,7 @@ linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, cons
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = m0 + wm + 16 * i + 4 * kl + r;
-                if (row < M) y[(size_t)row * N + col] = acc[i][j][r] + b;
+                if (row < M) y[(size_t)row * N + col] = (VEC ? sum : acc)[i][j][r] + b;
             }
     }
 }
@@ -117,7 +133,7 @@ linear_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, cons
 // Bound: HBM / L2 on w for few rows, fp32 MFMA for many.
 // ---------------------------------------------------------------------------
 constexpr int kLinRing = 2;
-// Cost rule of launch_direct: bytes per cycle a CU loads with 16 rows per
+// Cost rule of launch_vec: bytes per cycle a CU loads with 16 rows per
 // 16-lane group (measured: one such 1 KiB wave load per 64 cycles), and cycles
 // a tile costs besides (LDS sum, stores).
 constexpr double kLinLoadBytes = 15, kLinTileCycles = 1000;
@@ -273,36 +289,61 @@ void launch_tile(const float* x, const float* w, const float* bias, float* y, in
                        N % 4 == 0 && aligned16(y) ? 1 : 0);
 }
 
-// The tile with the smallest estimated time per CU: tiles per CU times the
-// larger of a tile's MFMA cycles (its waves share the CU's four SIMDs, 32
-// cycles per 16x16x4) and its load cycles, plus a tile's fixed cycles.
-// Measured (N, K = 3072, 1024; weights rotated over 75 MB), tiles 16x16 /
-// 16x32 / 32x32 / 32x64 / 64x64 against linear_f32_kernel, us: M = 1 4.8 / 6.6
-// / 8.6 / 13.7 / 22.5 against 48; M = 128 24 / 18.5 / 18.7 / 15.7 / 27 against
-// 53; M = 1024 169 / 128 / 101 / 92 / 78 against 80.  N, K = 2048, 6144: M = 1
-// 18 .. 107 against 354, M = 1024 673 .. 222 against 472.
-void launch_direct(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
-                   hipStream_t st) {
-    static constexpr int kTiles[][3] = {{16, 16, 8}, {16, 32, 8}, {32, 32, 8}, {32, 64, 4}, {64, 64, 4}};
+// K % 4 == 0, 16-byte aligned x and w.  Of the direct kernel's tiles, the one
+// with the smallest estimated time per CU: tiles per CU times the larger of a
+// tile's MFMA cycles (its waves share the CU's four SIMDs, 32 cycles per
+// 16x16x4) and its load cycles, plus a tile's fixed cycles.  That tile or
+// linear_f32_kernel, whichever has the smaller estimated microseconds (direct_us,
+// lds_us: fitted to 1684 sizes, M 1 .. 4096, N 16 .. 151936, K 32 .. 8192).  A
+// direct tile is one workgroup's serial course; the LDS kernel's workgroups
+// share a CU, so it is ahead where a CU has many tiles of a short K.
+//
+// Measured us, tiles 16x16 / 16x32 / 32x32 / 32x64 / 64x64 against the LDS
+// kernel.  N, K = 3072, 1024 (weights rotated over 75 MB): M = 1 4.8 / 6.6 / 8.6
+// / 13.7 / 22.5 against 48; M = 128 24 / 18.5 / 18.7 / 15.7 / 27 against 53;
+// M = 1024 170 / 130 / 103 / 93 / 81 against 81; M = 4096 64x64 304 against 250.
+// M = 1024, N = 4096: K = 32 19 / 22 / 17 / 14 / 20 against 8.8, K = 256 115 / 90 /
+// 59 / 35 / 36 against 28, K = 2048 64x64 171 against 185.  N, K = 151936, 1024:
+// M = 64 64x64 279 against 252, M = 512 2068 against 1638.
+struct DirectTile { int rows, cols, waves; double us, us_k; };   // us of a tile: us + us_k K
+constexpr DirectTile kDirectTiles[] = {{16, 16, 8, 0.24, 0.0034}, {16, 32, 8, 0.6, 0.00514}, {32, 32, 8, 0.85, 0.00733},
+                                       {32, 64, 4, 1.1, 0.0105}, {64, 64, 4, 3.6, 0.0168}};
+
+void launch_vec(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, hipStream_t st) {
     const long long cus = device_cu_count();
     int best = 4;
-    double best_t = INFINITY;
+    double best_t = INFINITY, direct_us = 0;
     for (int i = 0; i < 5; ++i) {
-        const long long tm = kTiles[i][0], tn = kTiles[i][1];
-        const long long rows = (M + tm - 1) / tm, cols = (N + tn - 1) / tn;
-        if (i < 4 && (rows > 65535 || cols * kTiles[i][2] * 64 > 0xffffffffLL)) continue;   // grid limits
+        const DirectTile& d = kDirectTiles[i];
+        const long long rows = ((long long)M + d.rows - 1) / d.rows, cols = ((long long)N + d.cols - 1) / d.cols;
+        if (i < 4 && (rows > 65535 || cols * d.waves * 64 > 0xffffffffLL)) continue;   // grid limits
         const long long per_cu = (rows * cols + cus - 1) / cus;
-        const double mfma = (double)(tm * tn) / 256 * K / 16 * 32, load = (double)(tm + tn) * K * 4 / kLinLoadBytes;
-        const double both = kTiles[i][2] == 4 ? 0.5 * std::min(mfma, load) : 0.0;   // one wave per SIMD: partly serial
+        const double mfma = (double)(d.rows * d.cols) / 256 * K / 16 * 32;
+        const double load = (double)(d.rows + d.cols) * K * 4 / kLinLoadBytes;
+        const double both = d.waves == 4 ? 0.5 * std::min(mfma, load) : 0.0;   // one wave per SIMD: partly serial
         const double t = per_cu * (std::max(mfma, load) + both + kLinTileCycles);
-        if (t < best_t) { best = i; best_t = t; }
+        if (t < best_t) {
+            best = i;
+            best_t = t;
+            double us = d.us + d.us_k * K;
+            if (i == 4) us += std::min(4.4, std::max(0.0036 * K, 0.009 * (K - 256)));   // beyond the loads in flight
+            if (i >= 3 && (double)N * K * 4 > 202e6) us *= 1.08;   // w not kept in the 256 MB cache
+            direct_us = per_cu * us;
+        }
     }
+    const dim3 grid((N + kLinTile - 1) / kLinTile, (M + kLinTile - 1) / kLinTile);
+    const double tiles = (double)grid.x * grid.y / cus;   // of the LDS kernel per CU
+    const double lds_us = 1.0 + 0.5 * tiles +
+                          K * std::max({0.0645, 0.044 + 0.012 * tiles, 0.0295 + 0.0155 * tiles, 0.0197 * tiles});
+    if (lds_us < direct_us) best = 5;
     switch (best) {
         case 0: return launch_tile<16, 16, 8>(x, w, bias, y, M, N, K, st);
         case 1: return launch_tile<16, 32, 8>(x, w, bias, y, M, N, K, st);
         case 2: return launch_tile<32, 32, 8>(x, w, bias, y, M, N, K, st);
         case 3: return launch_tile<32, 64, 4>(x, w, bias, y, M, N, K, st);
-        default: return launch_tile<64, 64, 4>(x, w, bias, y, M, N, K, st);
+        case 4: return launch_tile<64, 64, 4>(x, w, bias, y, M, N, K, st);
+        default:
+            hipLaunchKernelGGL(linear_f32_kernel<true>, grid, dim3(256), 0, st, x, w, bias, y, M, N, K);
     }
 }
 
@@ -328,9 +369,9 @@ extern "C" sa_status sa_linear_f32(const float* x, int M, int K, const float* w,
     if (grid.y > 65535u) return fail(SA_EINVAL, "M too large for one launch");
     hipStream_t st = as_stream(stream);
     if (K > 0 && K <= (1 << 30) && K % 4 == 0 && aligned16(x) && aligned16(w))
-        launch_direct(x, w, bias, y, M, N, K, st);
+        launch_vec(x, w, bias, y, M, N, K, st);
     else
-        hipLaunchKernelGGL(linear_f32_kernel, grid, dim3(256), 0, st, x, w, bias, y, M, N, K);
+        hipLaunchKernelGGL(linear_f32_kernel<false>, grid, dim3(256), 0, st, x, w, bias, y, M, N, K);
     SA_CHECK_LAUNCH();
     return SA_OK;
 }

@@ -134,3 +134,25 @@ def test_linear_non_finite_inputs_stay_in_their_rows_and_columns(sa, synth):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
     ok = np.isfinite(want)
     near(got[ok], want[ok], "finite part")
+
+
+@pytest.mark.parametrize("M,K,N,lds", [(1000, 132, 3000, True), (1100, 36, 4100, True), (65, 4, 70000, True),
+                                       (520, 1024, 12290, True), (700, 1028, 1100, False), (300, 2052, 4100, False)])
+def test_linear_kernel_of_many_tiles(sa, synth, M, K, N, lds):
+    """Many 64 x 64 tiles per CU of a short K take the kernel whose workgroups
+    share a CU: it adds the products of every 32 k up by themselves, in order, and
+    then to the sum, so that a call has the bits of the sum of its 32-wide
+    parts' calls.  Fewer tiles or a longer K take the LDS-free kernel's 64 x 64
+    tile, whose waves split K.  (256 CUs.)"""
+    x = torch.from_numpy(synth.normal(54, M + K, (M, K))).cuda()
+    w = torch.from_numpy(synth.normal(55, N + K, (N, K), 0.05)).cuda()
+    b = torch.from_numpy(synth.normal(56, N, (N,))).cuda()
+    buf = torch.full((M * N + 64,), 7.0, device="cuda")
+    y = buf[32:32 + M * N].view(M, N)
+    sa.linear(x, w, b, out=y)
+    near(y.cpu().numpy(), (x.double() @ w.double().T + b).cpu().numpy(), (M, K, N))
+    assert bool((buf[:32] == 7.0).all()) and bool((buf[32 + M * N:] == 7.0).all())
+    parts = torch.zeros(M, N, device="cuda")
+    for k in range(0, K, 32):
+        parts += sa.linear(x[:, k:k + 32].contiguous(), w[:, k:k + 32].contiguous())
+    assert torch.equal(parts + b, y) == lds
