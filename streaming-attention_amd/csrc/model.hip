@@ -451,6 +451,7 @@ Shapes shapes_of(const sa_qwen3_desc& d) {
 // Floats of the partial-sum buffer of a decode step or prompt of up to B rows: a
 // few-row step's q | k | v and its o and down splits, or 8 splits of the wider of
 // qkv and o / down for up to 128 rows (more rows take fewer), gate and up unsplit.
+// A step of n rows plans with part_floats(n), whatever the model's max_batch.
 size_t part_floats(const Shapes& s, size_t B) {
     const size_t few = std::min<size_t>(B, kFewRows) * (s.Nqkv + 2 * kFewSplit * s.H);
     return std::max({few, 8 * std::min<size_t>(B, 128) * std::max(s.Nqkv, s.H), B * std::max({s.Nqkv, s.H, 2 * s.I})});
@@ -826,9 +827,9 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
         BesideProjections gb;
         DecodeParts parts;     // few rows: the attention's unmerged partials
     };
-    const size_t part_n = part_floats(s, m->max_batch);
     auto make_rows = [&](int r0, int n, float* part, void* ws, size_t ws_bytes, hipStream_t on, bool beside) {
         float* o_part = part + (size_t)n * s.Nqkv;
+        const size_t part_n = part_floats(s, n);   // of the buffer's: splits (and rounding) follow from the rows alone
         Rows r{r0, n, part, ws, ws_bytes, on, {}, few_rows_fit(n, s.H), m->x + (size_t)r0 * s.H,
                m->x2 + (size_t)r0 * s.H, o_part, o_part + (size_t)kFewSplit * n * s.H,
                beside, plan_layer(s, n, part_n), plan_beside(s, n, part_n), {}};

@@ -306,3 +306,25 @@ def test_model_decode_merged_partials(sa, oracle, synth, lens, head_dim):
         assert rel_l2(got, want) <= 1e-5, t
     run_parity(sa, oracle, synth, cfg, 0.1, lens, 2, sa.SA_DTYPE_F32, 31 + len(lens), [3 + b for b in range(len(lens))],
                check)
+
+
+def test_model_decode_same_bits_at_any_max_batch(sa, synth, monkeypatch):
+    """The K splits of an interleaved half-batch of 256 rows, whose partials
+    limit them, follow from its rows: a model made for 512 rows and one
+    made for 1024 give the same bits."""
+    monkeypatch.setenv("SA_DECODE_INTERLEAVE", "1")
+    cfg = dict(SMALL, num_layers=1, hidden=1024, intermediate=1024, n_q_heads=8, n_kv_heads=4, vocab=256)
+    lens = [33] * 512
+    tokens = torch.tensor([(7 * i + 3) % cfg["vocab"] for i in range(len(lens))], dtype=torch.int32, device="cuda")
+    got = []
+    for max_batch in (512, 1024):
+        model = sa.Qwen3(max_batch, 64, **{k: cfg[k] for k in SHAPE_KEYS})
+        model.init_random(14, 0.1)
+        cache = make_cache(sa, synth, cfg, lens, 1, sa.SA_DTYPE_F32, 14)
+        logits = torch.empty(len(lens), cfg["vocab"], dtype=torch.float32, device="cuda")
+        model.decode_step(cache, tokens, logits=logits)
+        torch.cuda.synchronize()
+        got.append(logits)
+        cache.close()
+        model.close()
+    assert torch.equal(got[0], got[1])
