@@ -35,4 +35,10 @@ inline DecodeParts plan_parts(const float* ml, const float* o, int n_seq, int n_
     return p;
 }
 
+// Tokens that one launch of rows head rows per token takes, lanes threads each:
+// at most 2^31 threads (a launch has fewer than 2^32).
+inline int tokens_per_launch(int rows, int lanes) {
+    return (int)std::max<long long>(1, (1LL << 31) / ((long long)rows * lanes));
+}
+
 }  // namespace sa

@@ -579,11 +579,10 @@ sa_status append_impl(sa_kvcache* c, int layer, const float* q, const float* k, 
         for (const void* p : std::initializer_list<const void*>{a.q, a.k, a.v, a.part, a.q_out, a.k_out, a.v_out, a.wq,
                                                                 a.wk, a.cos_t, a.sin_t})
             vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-        // Tokens per launch: row indices and the grid stay within 31 bits.
-        const int step = std::max(1, (1 << 28) / rows);
+        const int lanes = std::min(D / 2, kWave) / 4;
+        const int step = tokens_per_launch(rows, lanes);
         for (a.s0 = 0; a.s0 < S; a.s0 += a.n_s) {
             a.n_s = std::min(step, S - a.s0);
-            const int lanes = std::min(D / 2, kWave) / 4;
             const dim3 grid((unsigned)(((long long)rows * a.n_s * lanes + 255) / 256), m);
             switch (D) {
 #define SA_APPEND_LAUNCH(DD, BB, VV)                                                                               \

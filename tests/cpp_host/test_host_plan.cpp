@@ -1,5 +1,6 @@
 // CPU unit test of the host-side launch planning (csrc/host_plan.h; no GPU, no
-// HIP): the partials a decode launch leaves to its consumer.
+// HIP): the partials a decode launch leaves to its consumer, the tokens of an
+// append's launch.
 #include "host_plan.h"
 
 #include <cstdio>
@@ -53,6 +54,12 @@ int main() {
                     check_rows(n, longest, chunk, longest - 1 > 0 ? longest - 1 : 1);   // a full table row
                 }
     }
+    for (int lanes : {1, 2, 4, 8, 16, 32, 64})
+        for (int rows : {2, 3, 24, 32, 48, 64, 1000, 1 << 20}) {
+            const long long t = sa::tokens_per_launch(rows, lanes);
+            EXPECT(t >= 1 && t * rows * lanes <= 1LL << 31);          // threads of a launch
+            EXPECT((t + 1) * rows * lanes > 1LL << 31);               // as many as fit
+        }
     if (g_fail) return 1;
     std::printf("all checks passed\n");
     return 0;

@@ -1,7 +1,8 @@
 """CPU test of the host-side launch planning (csrc/host_plan.h): the C++ unit
 test in tests/cpp_host is compiled with g++ (no HIP) and run.  It covers the
 partials a decode launch leaves to its consumer for 1 to 16 rows, with guard
-words around the plan."""
+words around the plan, and the tokens of one launch of an append, whose threads
+stay below a launch's limit."""
 from __future__ import annotations
 
 import shutil
