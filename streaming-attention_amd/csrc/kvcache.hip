@@ -101,13 +101,14 @@ sa_status publish_lens(sa_kvcache* c, const int32_t* rows, int n, int val, int a
 sa_status refused(const Verdict& v) { return fail(v.status, v.msg); }
 
 // ---------------------------------------------------------------------------
-// Fused QK-norm + RoPE + append.  A head row (query, key or value) is served by
-// D/8 lanes (16 at most), 16 bytes of each half per lane, so RoPE needs no lane
-// exchange and a wave moves 4 rows of 128 elements per load.
+// Fused QK-norm + RoPE + append.  A head row (query, key or value) of a prompt is
+// served by D/8 lanes (16 at most), 16 bytes of each half per lane, so RoPE needs
+// no lane exchange and a wave moves 4 rows of 128 elements per load; the rows of a
+// small launch by D/2 lanes (64 at most; kAppendNarrow).
 //
-// Bound: the 21 MB of 1024 tokens (16 query and 8 KV heads of 128, bf16 cache)
-// at HBM rate are 3.3 us of a launch.  Rows of 64 lanes with 4-byte loads took
-// 8.8 us: twice the waves, each with four loads of 256 bytes in flight.
+// Bound: HBM for prompts: the 29.4 MB of 1024 tokens (16 query and 8 KV heads of
+// 128, bf16 cache) take 4.7 us at 6.3 TB/s; the launch takes 7.1 us, 4096 tokens
+// 22.5 (rows of 64 lanes with 4-byte loads, two per wave of keys: 7.9 and 25.1).
 // ---------------------------------------------------------------------------
 struct AppendArgs {
     const float* q; const float* k; const float* v;
@@ -145,39 +146,40 @@ qk_norm_rope_kernel(const float* x, int n_rows, const int32_t* pos, const float*
     r.store(y + (size_t)row * D, lane);
 }
 
-// A head row over LANES lanes: lane j holds elements i .. i + 3 and their
-// rotate-half partners i + D/2 .. for i = 4 j + 64 c.  The arithmetic is RowPairs'
-// (the same sums in the same order), so both give the same bits.
-template <int D, bool VEC>
-struct RowQuads {
+// A head row over LANES lanes: lane j holds elements i .. i + E - 1 and their
+// rotate-half partners i + D/2 .. for i = E j + 64 c.  The arithmetic is RowPairs'
+// (the same sums in the same order), so all give the same bits.
+template <int D, int E, bool VEC>
+struct LaneRow {
+    static_assert(E == 4 || (E == 1 && !VEC), "one or four elements");
     static constexpr int H = D / 2;
-    static constexpr int LANES = (H < kWave ? H : kWave) / 4;
+    static constexpr int LANES = (H < kWave ? H : kWave) / E;
     static constexpr int NC = (H + kWave - 1) / kWave;
-    float lo[NC][4], hi[NC][4];
+    float lo[NC][E], hi[NC][E];
 
-    // 4 floats; VEC: 16-byte aligned.
-    __device__ static __forceinline__ void load4(const float* x, float (&v)[4]) {
+    // E floats; VEC: 16-byte aligned.
+    __device__ static __forceinline__ void load_e(const float* x, float (&v)[E]) {
         if constexpr (VEC) {
             const float4 f = *reinterpret_cast<const float4*>(x);
             v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = x[e];
+            for (int e = 0; e < E; ++e) v[e] = x[e];
         }
     }
-    __device__ static __forceinline__ void store4(float* y, const float (&v)[4]) {
+    __device__ static __forceinline__ void store_e(float* y, const float (&v)[E]) {
         if constexpr (VEC) {
             *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = v[e];
+            for (int e = 0; e < E; ++e) y[e] = v[e];
         }
     }
     __device__ __forceinline__ void load(const float* x, int j) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            load4(x + 4 * j + kWave * c, lo[c]);
-            load4(x + 4 * j + kWave * c + H, hi[c]);
+            load_e(x + E * j + kWave * c, lo[c]);
+            load_e(x + E * j + kWave * c + H, hi[c]);
         }
     }
     // The sum, in split order, of S split-K partial rows x[t * split] ...
@@ -185,15 +187,15 @@ struct RowQuads {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) lo[c][e] = hi[c][e] = 0.f;
+            for (int e = 0; e < E; ++e) lo[c][e] = hi[c][e] = 0.f;
 #pragma unroll 4
         for (int t = 0; t < S; ++t) {
-            RowQuads p;
+            LaneRow p;
             p.load(x + t * split, j);
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
+                for (int e = 0; e < E; ++e) {
                     lo[c][e] += p.lo[c][e];
                     hi[c][e] += p.hi[c][e];
                 }
@@ -201,19 +203,21 @@ struct RowQuads {
     }
     __device__ __forceinline__ void rms_norm(const float* w, float eps, int j) {
 #pragma clang fp contract(off)
-        RowQuads g;
+        LaneRow g;
         g.load(w, j);
-        float t[4] = {0.f, 0.f, 0.f, 0.f};
+        float t[E] = {};
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) t[e] = fmaf(lo[c][e], lo[c][e], fmaf(hi[c][e], hi[c][e], t[e]));
-        const float ss = group_reduce<OpSum, 1, LANES>((t[0] + t[1]) + (t[2] + t[3]));
+            for (int e = 0; e < E; ++e) t[e] = fmaf(lo[c][e], lo[c][e], fmaf(hi[c][e], hi[c][e], t[e]));
+        float ss = t[0];
+        if constexpr (E == 4) ss = (t[0] + t[1]) + (t[2] + t[3]);
+        ss = group_reduce<OpSum, 1, LANES>(ss);
         const float rms = sqrtf(ss / (float)D + eps);
 #pragma unroll
         for (int c = 0; c < NC; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < E; ++e) {
                 lo[c][e] = (lo[c][e] / rms) * g.lo[c][e];
                 hi[c][e] = (hi[c][e] / rms) * g.hi[c][e];
             }
@@ -222,11 +226,11 @@ struct RowQuads {
 #pragma clang fp contract(off)
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            float cs[4], sn[4];
-            load4(cos_t + (size_t)pos * H + 4 * j + kWave * c, cs);
-            load4(sin_t + (size_t)pos * H + 4 * j + kWave * c, sn);
+            float cs[E], sn[E];
+            load_e(cos_t + (size_t)pos * H + E * j + kWave * c, cs);
+            load_e(sin_t + (size_t)pos * H + E * j + kWave * c, sn);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < E; ++e) {
                 const float l2 = lo[c][e] * cs[e] - hi[c][e] * sn[e];
                 const float h2 = hi[c][e] * cs[e] + lo[c][e] * sn[e];
                 lo[c][e] = l2;
@@ -237,40 +241,51 @@ struct RowQuads {
     __device__ __forceinline__ void store(float* y, int j) const {
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            store4(y + 4 * j + kWave * c, lo[c]);
-            store4(y + 4 * j + kWave * c + H, hi[c]);
+            store_e(y + E * j + kWave * c, lo[c]);
+            store_e(y + E * j + kWave * c + H, hi[c]);
         }
     }
     // A row of the cache pools, 16-byte aligned.
     template <bool BF16>
     __device__ __forceinline__ void store_pool(char* pool, size_t row, int j) const {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const size_t i = row + 4 * j + kWave * c;
-            if constexpr (BF16) {
-                auto put = [&](size_t at, const float (&v)[4]) {
+        if constexpr (BF16) {
+            uint16_t* d = reinterpret_cast<uint16_t*>(pool) + row;
+            auto put = [&](int at, const float (&v)[E]) {
+                if constexpr (E == 4) {
                     uint32_t b[2];
 #pragma unroll
                     for (int e = 0; e < 2; ++e)
                         b[e] = f32_to_bf16_rne(v[2 * e]) | (uint32_t)f32_to_bf16_rne(v[2 * e + 1]) << 16;
-                    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(pool) + at) = make_uint2(b[0], b[1]);
-                };
-                put(i, lo[c]);
-                put(i + H, hi[c]);
-            } else {
-                float* d = reinterpret_cast<float*>(pool);
-                *reinterpret_cast<float4*>(d + i) = make_float4(lo[c][0], lo[c][1], lo[c][2], lo[c][3]);
-                *reinterpret_cast<float4*>(d + i + H) = make_float4(hi[c][0], hi[c][1], hi[c][2], hi[c][3]);
+                    *reinterpret_cast<uint2*>(d + at) = make_uint2(b[0], b[1]);
+                } else {
+                    d[at] = f32_to_bf16_rne(v[0]);
+                }
+            };
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                put(E * j + kWave * c, lo[c]);
+                put(E * j + kWave * c + H, hi[c]);
+            }
+        } else {
+            float* d = reinterpret_cast<float*>(pool) + row;
+            auto put = [&](int at, const float (&v)[E]) {
+                if constexpr (E == 4) *reinterpret_cast<float4*>(d + at) = make_float4(v[0], v[1], v[2], v[3]);
+                else d[at] = v[0];
+            };
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                put(E * j + kWave * c, lo[c]);
+                put(E * j + kWave * c + H, hi[c]);
             }
         }
     }
 };
 
 // VEC: q, k, v, the partials, weights, tables and outputs are 16-byte aligned.
-template <int D, bool BF16, bool VEC>
+template <int D, bool BF16, int E, bool VEC>
 __global__ void __launch_bounds__(256)
 qknorm_rope_append_kernel(AppendArgs a) {
-    using Row = RowQuads<D, VEC>;
+    using Row = LaneRow<D, E, VEC>;
     const int j = threadIdx.x % Row::LANES;
     const unsigned idx = blockIdx.x * (256u / Row::LANES) + threadIdx.x / Row::LANES;
     const unsigned per_token = a.n_q + 2 * a.n_kv;
@@ -538,6 +553,14 @@ namespace sa {
 
 namespace {
 
+// Head rows of a launch up to which a row takes 64 lanes (at most 12 waves a CU
+// of 256): alone a launch is the latency of one row, and eight divisions per
+// lane are a longer chain than two.  us, 64 lanes / 16 / the launch of one wave
+// per query or key-and-value row before: 64 sequences of one token, bf16 cache,
+// 2.55 / 3.06 / 2.66, 64 tokens 2.56 / 2.87 / 2.65, 128 tokens (4096 rows) 2.93 / 2.94 /
+// 2.91, 256 tokens 3.99 / 3.50 / 3.57, 1024 tokens 10.6 / 7.1 / 7.9.
+constexpr long long kAppendNarrow = 3000;
+
 // Shared by the entry points below: q/k/v given (part == NULL), or summed from
 // the n_part split-K partials of the projection at part (q, k, v NULL).
 sa_status append_impl(sa_kvcache* c, int layer, const float* q, const float* k, const float* v, const float* part,
@@ -575,24 +598,27 @@ sa_status append_impl(sa_kvcache* c, int layer, const float* q, const float* k, 
         a.v = v ? v + (size_t)i0 * S * a.n_kv * D : nullptr;
         a.v_out = v_out ? v_out + (size_t)i0 * S * a.n_kv * D : nullptr;
         a.part_row0 = i0 * S;
-        bool vec = true;   // the launch's pointers allow 16-byte accesses
+        const bool wide = (long long)rows * S * m > kAppendNarrow;
+        bool vec = wide;   // the launch's pointers allow 16-byte accesses
         for (const void* p : std::initializer_list<const void*>{a.q, a.k, a.v, a.part, a.q_out, a.k_out, a.v_out, a.wq,
                                                                 a.wk, a.cos_t, a.sin_t})
-            vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-        const int lanes = std::min(D / 2, kWave) / 4;
+            vec = vec && aligned16(p);
+        const int lanes = std::min(D / 2, kWave) / (wide ? 4 : 1);
         const int step = tokens_per_launch(rows, lanes);
         for (a.s0 = 0; a.s0 < S; a.s0 += a.n_s) {
             a.n_s = std::min(step, S - a.s0);
             const dim3 grid((unsigned)(((long long)rows * a.n_s * lanes + 255) / 256), m);
             switch (D) {
-#define SA_APPEND_LAUNCH(DD, BB, VV)                                                                               \
-    hipLaunchKernelGGL((qknorm_rope_append_kernel<DD, BB, VV>), grid, dim3(256), 0, st, a)
+#define SA_APPEND_LAUNCH(DD, BB, EE, VV)                                                                           \
+    hipLaunchKernelGGL((qknorm_rope_append_kernel<DD, BB, EE, VV>), grid, dim3(256), 0, st, a)
 #define SA_APPEND_CASE(DD)                                                                                         \
     case DD:                                                                                                       \
-        if (bf && vec) SA_APPEND_LAUNCH(DD, true, true);                                                           \
-        else if (bf) SA_APPEND_LAUNCH(DD, true, false);                                                            \
-        else if (vec) SA_APPEND_LAUNCH(DD, false, true);                                                           \
-        else SA_APPEND_LAUNCH(DD, false, false);                                                                   \
+        if (bf && vec) SA_APPEND_LAUNCH(DD, true, 4, true);                                                        \
+        else if (bf && wide) SA_APPEND_LAUNCH(DD, true, 4, false);                                                 \
+        else if (bf) SA_APPEND_LAUNCH(DD, true, 1, false);                                                         \
+        else if (vec) SA_APPEND_LAUNCH(DD, false, 4, true);                                                        \
+        else if (wide) SA_APPEND_LAUNCH(DD, false, 4, false);                                                      \
+        else SA_APPEND_LAUNCH(DD, false, 1, false);                                                                \
         break;
                 SA_APPEND_CASE(8)
                 SA_APPEND_CASE(16)

@@ -512,13 +512,8 @@ def test_cache_on_nonblocking_stream(sa, oracle, synth):
     cache.close()
 
 
-@pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("d", [8, 16, 32, 64, 128, 256])
-def test_append_equals_standalone_norm_rope(sa, d, shift, bf16):
-    """A prompt's append over ragged row counts, from 16-byte aligned pointers
-    and from pointers 4 bytes past: the bits of the standalone norm + RoPE."""
-    B, S, hq, hkv, eps = 2, 67, 6, 3, 1e-6
+def append_equals_standalone(sa, d, shift, bf16, S):
+    B, hq, hkv, eps, pages = 2, 6, 3, 1e-6, (S + 63) // 64
     gen = torch.Generator(device="cuda").manual_seed(d + shift)
 
     def rand(*shape):
@@ -527,9 +522,9 @@ def test_append_equals_standalone_norm_rope(sa, d, shift, bf16):
     q, k, v = rand(B, S, hq, d), rand(B, S, hkv, d), rand(B, S, hkv, d)
     wq, wk = rand(d), rand(d)
     rope = tuple(rand(S, d // 2).copy_(t) for t in sa.rope_tables(S, d, 1e6))
-    cache = sa.KVCache(1, hkv, d, B, 2, 4, sa.SA_DTYPE_BF16 if bf16 else sa.SA_DTYPE_F32)
+    cache = sa.KVCache(1, hkv, d, B, pages, B * pages, sa.SA_DTYPE_BF16 if bf16 else sa.SA_DTYPE_F32)
     for s in range(B):
-        cache.set_pages(s, [3 - 2 * s, 2 - 2 * s])
+        cache.set_pages(s, [B * pages - 1 - pages * s - p for p in range(pages)])
     q_out = rand(B, S, hq, d)
     cache.append(0, q, k, v, wq, wk, eps, rope, q_out=q_out)
     cache.commit(S, n_seqs=B)
@@ -546,3 +541,21 @@ def test_append_equals_standalone_norm_rope(sa, d, shift, bf16):
             ref = ref.transpose(0, 1)
             assert torch.equal(got, ref.bfloat16().float() if bf16 else ref)
     cache.close()
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("d", [8, 16, 32, 64, 128, 256])
+def test_append_equals_standalone_norm_rope(sa, d, shift, bf16):
+    """A prompt's append over ragged row counts, from 16-byte aligned pointers
+    and from pointers 4 bytes past: the bits of the standalone norm + RoPE."""
+    append_equals_standalone(sa, d, shift, bf16, 67)
+
+
+# 12 head rows a token and two sequences: 64 lanes a row up to 3000 rows, which
+# 125 tokens just fill, 16 above; the last launch ends inside a workgroup.
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("d,S", [(8, 131), (16, 300), (32, 127), (64, 126), (128, 125), (128, 126), (256, 203)])
+def test_append_of_more_rows_equals_standalone(sa, d, S, shift, bf16):
+    append_equals_standalone(sa, d, shift, bf16, S)
