@@ -164,11 +164,17 @@ def _stream(stream) -> int | None:
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else stream
 
 
+_float32 = None   # torch.float32 (torch is imported by the first call that needs it)
+
+
 def _f32(t, name: str):
-    import torch
+    global _float32
     if t is None:
         return None
-    if t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous():
+    if _float32 is None:
+        import torch
+        _float32 = torch.float32
+    if t.dtype != _float32 or not t.is_cuda or not t.is_contiguous():
         raise ValueError(f"{name} must be a contiguous float32 CUDA tensor")
     return t
 
