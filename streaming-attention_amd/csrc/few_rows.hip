@@ -404,22 +404,26 @@ bool few_rows_fit(int rows, int hidden) {
 namespace {
 
 // One instantiation per power of two of row pairs: the row loads are
-// unconditional.  Merged rows: at most 8 partials over a wave's row pairs
-// (more spill the 128 registers that 16 waves leave), as parts_limit says.
+// unconditional.  Merged rows: at most kPartsMax partials over a wave's row
+// pairs (more spill the 128 registers that 16 waves leave), as parts_limit says.
 template <int W, int PRO, int EPI, int NS = 0>
 sa_status launch_rows(const FewArgs& a, dim3 grid, hipStream_t st) {
-    const dim3 block(W * 64);
-    auto launch = [&](auto rp) {
+    auto launch = [&](auto rp) -> sa_status {
         constexpr int RP = decltype(rp)::value;
-        if constexpr (RP * NS <= kPartsMax)
-            hipLaunchKernelGGL((few_rows_kernel<W, RP, PRO, EPI, NS>), grid, block, 0, st, a);
+        if constexpr (RP * NS <= kPartsMax) {
+            hipLaunchKernelGGL((few_rows_kernel<W, RP, PRO, EPI, NS>), grid, dim3(W * 64), 0, st, a);
+            SA_CHECK_LAUNCH();
+            return SA_OK;
+        } else {
+            return fail(SA_EINVAL, "no launch merges this many partials of this many rows");
+        }
     };
-    if (a.M <= 2) launch(std::integral_constant<int, 1>{});
-    else if (a.M <= 4) launch(std::integral_constant<int, 2>{});
-    else if (a.M <= 8) launch(std::integral_constant<int, 4>{});
-    else launch(std::integral_constant<int, 8>{});
-    SA_CHECK_LAUNCH();
-    return SA_OK;
+    switch (row_pairs(a.M)) {
+        case 1: return launch(std::integral_constant<int, 1>{});
+        case 2: return launch(std::integral_constant<int, 2>{});
+        case 4: return launch(std::integral_constant<int, 4>{});
+        default: return launch(std::integral_constant<int, 8>{});
+    }
 }
 
 }  // namespace
@@ -440,10 +444,12 @@ sa_status few_project_split(const float* x, int M, int K, const uint16_t* W, int
     if (parts->n_split > parts_limit(M)) return fail(SA_EINVAL, "more partials than the rows can merge");
     a.parts = *parts;
     a.d_log2 = __builtin_ctz(D);
-    if (parts->n_split <= 2) return launch_rows<16, kPlain, kOut, 2>(a, grid, st);
-    if (parts->n_split <= 4) return launch_rows<16, kPlain, kOut, 4>(a, grid, st);
-    if (parts->n_split <= 6) return launch_rows<16, kPlain, kOut, 6>(a, grid, st);
-    return launch_rows<16, kPlain, kOut, kPartsMax>(a, grid, st);
+    switch (parts_form(parts->n_split)) {
+        case 2: return launch_rows<16, kPlain, kOut, 2>(a, grid, st);
+        case 4: return launch_rows<16, kPlain, kOut, 4>(a, grid, st);
+        case 6: return launch_rows<16, kPlain, kOut, 6>(a, grid, st);
+        default: return launch_rows<16, kPlain, kOut, kPartsMax>(a, grid, st);
+    }
 }
 
 sa_status few_head(const FewInput& in, int M, int K, const uint16_t* W, int N, float* logits, float* am_val,

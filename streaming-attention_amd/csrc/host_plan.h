@@ -21,7 +21,11 @@ struct DecodeParts {
 };
 
 // The most partials per row that M rows' consumer holds in registers.
-inline int parts_limit(int M) { return M <= 2 ? 8 : M <= 4 ? 4 : M <= kPartsRows ? 2 : 1; }
+constexpr int parts_limit(int M) { return M <= 2 ? 8 : M <= 4 ? 4 : M <= kPartsRows ? 2 : 1; }
+// The forms of that consumer: row pairs it has registers for, and partials
+// per row.  A form exists where the two multiply to at most kPartsMax.
+constexpr int row_pairs(int M) { return M <= 2 ? 1 : M <= 4 ? 2 : M <= 8 ? 4 : 8; }
+constexpr int parts_form(int n) { return n <= 2 ? 2 : n <= 4 ? 4 : n <= 6 ? 6 : kPartsMax; }
 
 // The partials that a launch of n_seq rows in n_split chunks leaves to its
 // consumer: those of at most parts_limit chunks, so of at most kPartsRows rows.

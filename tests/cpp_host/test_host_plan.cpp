@@ -47,6 +47,10 @@ int main() {
     for (int n = 1; n <= 16; ++n) {
         EXPECT(sa::parts_limit(n) >= 1 && sa::parts_limit(n) <= sa::kPartsMax);
         EXPECT(n <= sa::kPartsRows || sa::parts_limit(n) == 1);
+        // every count up to the limit has a form that holds it
+        EXPECT(2 * sa::row_pairs(n) >= n);
+        for (int s = 2; s <= sa::parts_limit(n); ++s)
+            EXPECT(sa::parts_form(s) >= s && sa::parts_form(s) * sa::row_pairs(n) <= sa::kPartsMax);
         for (int chunk : {64, 128, 256, 4096})
             for (int chunks = 1; chunks <= 10; ++chunks)
                 for (int longest : {chunk * (chunks - 1) + 1, chunk * chunks}) {

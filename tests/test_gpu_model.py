@@ -292,7 +292,7 @@ def test_model_decode_few_rows(sa, oracle, synth, interleave, rows, hidden, inte
 
 # Partials merged by the o projection: 2 .. 8 chunks of 128 tokens for up to
 # 2 rows, 4 for up to 4, 2 for up to 8, beside rows of one chunk; one chunk
-# more than the limit takes the merge launch.
+# more takes chunks of 256 tokens, still merged there.
 @pytest.mark.parametrize("lens", [[130], [1023], [1024], [30, 600], [257, 127, 510], [512, 5, 1, 300], [511, 513, 64, 9],
                                   [255, 3, 200, 128, 127], [100, 129, 254, 17, 64, 250, 1, 255], [256] * 7])
 @pytest.mark.parametrize("head_dim", [64, 128])
@@ -305,6 +305,24 @@ def test_model_decode_merged_partials(sa, oracle, synth, lens, head_dim):
         assert np.abs(got - want).max() <= 1e-4, t
         assert rel_l2(got, want) <= 1e-5, t
     run_parity(sa, oracle, synth, cfg, 0.1, lens, 2, sa.SA_DTYPE_F32, 31 + len(lens), [3 + b for b in range(len(lens))],
+               check)
+
+
+# The most chunks of 256 tokens that the o projection merges (8 of up to 2
+# rows, 4 of up to 4, 2 of up to 8) and one more, which takes the merge launch,
+# as two chunks of more than 8 rows do: each step below adds a token.
+@pytest.mark.parametrize("lens", [[2046], [2047], [9, 2047], [5, 1023, 700], [1024, 1, 90, 300], [511, 3, 200, 128, 127],
+                                  [100, 129, 254, 17, 64, 512, 1, 255], [255] + [7 * i + 1 for i in range(8)],
+                                  [600] + [9 * i + 1 for i in range(8)], [30 * i + 5 for i in range(15)] + [256]])
+def test_model_decode_past_merged_partials(sa, oracle, synth, lens):
+    """fp32 KV: as test_model_decode_fp32_kv, at the limit of the chunks the o
+    projection merges and past it."""
+    cfg = dict(SMALL, num_layers=1)
+
+    def check(t, got, want):
+        assert np.abs(got - want).max() <= 1e-4, t
+        assert rel_l2(got, want) <= 1e-5, t
+    run_parity(sa, oracle, synth, cfg, 0.1, lens, 2, sa.SA_DTYPE_F32, 51 + len(lens), [3 + b for b in range(len(lens))],
                check)
 
 
