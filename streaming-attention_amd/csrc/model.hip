@@ -85,6 +85,15 @@ constexpr int kArgBlocks = 64;   // argmax workgroups per row
 // A decode step interleaves two half-batches when the attention streams at
 // least this many cached K/V bytes per layer.
 constexpr long long kInterleaveBytes = 1LL << 30;
+// Cached bytes per layer from which an interleaved half-batch of at most kFewRows
+// rows takes the GEMM of many rows (see gemm_xwt_kernel): its 30 KiB of LDS fit
+// beside the other half's attention, the few-row launches' 40 to 155 KiB do not,
+// and once the attention outlasts them that costs more than their fewer
+// launches save.  28 layers, few-row launches against the GEMM: 1.3 GB (32
+// sequences of 10,000 tokens, bf16) 6.89 / 7.21 ms, 1.6 GB (12,000) 7.99 / 8.23, 1.8 GB
+// (14,000) 8.98 / 8.87, 2.1 GB (8,000, fp32) 10.14 / 9.73, 2.5 GB (16 of 38,000, bf16)
+// 11.44 / 11.08, 3.9 GB (24 of 20,000, fp32) 17.58 / 17.07.
+constexpr long long kBesideBytes = (1LL << 30) * 17 / 10;
 
 // ---------------------------------------------------------------------------
 // Synthetic weights: the splitmix64 / Box-Muller generator of the test
@@ -807,6 +816,27 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     const float eps = d.rms_eps;
     const float scale = 1.0f / sqrtf((float)d.head_dim);
     float* out_logits = logits ? logits : m->logits;
+    // Interleaving: with enough context, the batch runs as two half-batches
+    // on two streams, the second starting its first attention when the
+    // first half's ends.  From then on the halves run free, half a layer
+    // apart: each half's projections, norms and MLP (latency-bound launches)
+    // run while the other half's attention streams the cache, and each
+    // attention launch's tail overlaps the other's.  The halves split the
+    // cached tokens evenly; SA_DECODE_INTERLEAVE=0 / 1 forces it off / on.
+    // Measured on the 28-layer, 64-sequence bf16 step (979-31,078 tokens,
+    // same box): 19.61 ms against 20.48 ms on one stream; with the halves'
+    // attention launches strictly alternating (an event wait before each),
+    // 20.78 ms: a cross-stream wait costs ~12 us and each half-batch launch
+    // has a tail of its own.
+    long long total = 0;
+    std::vector<long long> prefix(M + 1, 0);
+    for (int i = 0; i < M; ++i) prefix[i + 1] = prefix[i] + sa_kvcache_len(cache, i) + 1;
+    total = prefix[M];
+    const int kv_elem = kd.kv_dtype == SA_DTYPE_BF16 ? 2 : 4;
+    const long long attn_bytes = total * d.n_kv_heads * d.head_dim * 2LL * kv_elem;
+    const char* fenv = std::getenv("SA_DECODE_INTERLEAVE");
+    const bool interleave = M >= 2 && (fenv ? std::atoi(fenv) != 0 : attn_bytes >= kInterleaveBytes);
+    const bool long_attn = attn_bytes >= kBesideBytes;
     bool few_head_rows = false;   // the head takes the last layer's residual sum of all rows
 
     // Rows [r0, r0 + n) of the batch on one stream: its own split-K partials
@@ -830,7 +860,7 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     auto make_rows = [&](int r0, int n, float* part, void* ws, size_t ws_bytes, hipStream_t on, bool beside) {
         float* o_part = part + (size_t)n * s.Nqkv;
         const size_t part_n = part_floats(s, n);   // of the buffer's: splits (and rounding) follow from the rows alone
-        Rows r{r0, n, part, ws, ws_bytes, on, {}, few_rows_fit(n, s.H), m->x + (size_t)r0 * s.H,
+        Rows r{r0, n, part, ws, ws_bytes, on, {}, few_rows_fit(n, s.H) && !(beside && long_attn), m->x + (size_t)r0 * s.H,
                m->x2 + (size_t)r0 * s.H, o_part, o_part + (size_t)kFewSplit * n * s.H,
                beside, plan_layer(s, n, part_n), plan_beside(s, n, part_n), {}};
         for (int i = 0; i < n; ++i) r.ids.push_back(r0 + i);
@@ -905,26 +935,6 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     hipLaunchKernelGGL(embed_norm_kernel, dim3(M), dim3(256), 0, st, m->embed, tokens, s.V, s.H,
                        m->layers[0].in_norm, eps, m->x, m->h);
     SA_CHECK_LAUNCH();
-    // Interleaving: with enough context, the batch runs as two half-batches
-    // on two streams, the second starting its first attention when the
-    // first half's ends.  From then on the halves run free, half a layer
-    // apart: each half's projections, norms and MLP (latency-bound launches)
-    // run while the other half's attention streams the cache, and each
-    // attention launch's tail overlaps the other's.  The halves split the
-    // cached tokens evenly; SA_DECODE_INTERLEAVE=0 / 1 forces it off / on.
-    // Measured on the 28-layer, 64-sequence bf16 step (979-31,078 tokens,
-    // same box): 19.61 ms against 20.48 ms on one stream; with the halves'
-    // attention launches strictly alternating (an event wait before each),
-    // 20.78 ms: a cross-stream wait costs ~12 us and each half-batch launch
-    // has a tail of its own.
-    long long total = 0;
-    std::vector<long long> prefix(M + 1, 0);
-    for (int i = 0; i < M; ++i) prefix[i + 1] = prefix[i] + sa_kvcache_len(cache, i) + 1;
-    total = prefix[M];
-    const int kv_elem = kd.kv_dtype == SA_DTYPE_BF16 ? 2 : 4;
-    const long long attn_bytes = total * d.n_kv_heads * d.head_dim * 2LL * kv_elem;
-    const char* fenv = std::getenv("SA_DECODE_INTERLEAVE");
-    const bool interleave = M >= 2 && (fenv ? std::atoi(fenv) != 0 : attn_bytes >= kInterleaveBytes);
     Rows all = make_rows(0, M, m->part, m->ws, m->ws_bytes, st, false);
     few_head_rows = all.few && !interleave;
     if (!interleave) {

@@ -326,6 +326,34 @@ def test_model_decode_past_merged_partials(sa, oracle, synth, lens):
                check)
 
 
+@pytest.mark.parametrize("tokens", [52000, 57500])
+def test_model_decode_interleaved_long_contexts(sa, synth, monkeypatch, tokens):
+    """Interleaved half-batches of few rows on either side of the 1.8 GB of
+    cached K/V per layer from which they take the GEMM of many rows: the
+    logits of the step on one stream (fp32; other sums in other orders)."""
+    cfg = dict(SMALL, num_layers=1, n_q_heads=8, n_kv_heads=8, head_dim=128)
+    lens = [tokens, tokens - 700, tokens + 33, tokens - 1]
+    model = sa.Qwen3(len(lens), max(lens) + 2, **{k: cfg[k] for k in SHAPE_KEYS})
+    model.init_random(15, 0.1)
+    cache = make_cache(sa, synth, cfg, lens, 2, sa.SA_DTYPE_F32, 15)
+    first = torch.tensor([3, 5, 7, 11], dtype=torch.int32, device="cuda")
+    got = []
+    for interleave in ("0", None):   # None: by the cached bytes, 1.7 GB and more
+        if interleave:
+            monkeypatch.setenv("SA_DECODE_INTERLEAVE", interleave)
+        else:
+            monkeypatch.delenv("SA_DECODE_INTERLEAVE")
+        logits = torch.empty(len(lens), cfg["vocab"], dtype=torch.float32, device="cuda")
+        model.decode_step(cache, first, logits=logits)
+        torch.cuda.synchronize()
+        got.append(logits.cpu().numpy())
+        for i, n in enumerate(lens):
+            cache.set_len(i, n)
+    assert np.isfinite(got[0]).all() and rel_l2(got[1], got[0]) <= 1e-5
+    cache.close()
+    model.close()
+
+
 def test_model_decode_same_bits_at_any_max_batch(sa, synth, monkeypatch):
     """The K splits of an interleaved half-batch of 256 rows, whose partials
     limit them, follow from its rows: a model made for 512 rows and one
