@@ -1004,7 +1004,7 @@ sa_status decode_paged_fused(const PagedView& c, const float* q, int n_seq, cons
     // Partials that the consumer merges cost no launch: the smallest chunks, one
     // tile per wave, while it takes that many and they are one round of
     // workgroups.  28 layers, one sequence of 513 - 613 tokens: 11.0 ->
-    // 8.4 us of attention per layer, 1010 -> 962 us per step.
+    // 8.4 us of attention per layer, 1010 -> 975 us per step.
     const int small = (max_len + kMinChunk - 1) / kMinChunk;
     if (f.parts && forced_chunk() <= 0 && a.chunk > kMinChunk && small <= parts_limit(n_seq) &&
         (long long)small * c.n_kv * n_seq <= device_cu_count())

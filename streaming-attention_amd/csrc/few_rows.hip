@@ -265,8 +265,6 @@ struct HeadArgs {
     int M, K, N;
 };
 
-__device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
-
 __global__ void __launch_bounds__(kHeadWaves * 64)
 few_head_kernel(HeadArgs a) {
     extern __shared__ __align__(16) unsigned char terms[];   // [kTerms][kFewRows][K + 8] bf16

@@ -368,8 +368,6 @@ __global__ void __launch_bounds__(256) swiglu_kernel(const float* P, int S, int 
 // ---------------------------------------------------------------------------
 // Greedy argmax over the vocabulary (lowest index among equal maxima).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
-
 __device__ __forceinline__ void block_argmax(float& v, int& idx, float* sv, int* si) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
@@ -612,7 +610,8 @@ extern "C" sa_status sa_qwen3_create(const sa_qwen3_desc* desc, int max_batch, s
     if ((st = sa_rope_table_init(m->rope_cos, m->rope_sin, d.max_pos, d.head_dim, d.rope_theta, nullptr)) != SA_OK)
         return cleanup(st);
     const size_t part = part_floats(s, B), am = B * std::max(kArgBlocks, kFewHeadBlocks);
-    if ((st = dev_alloc(m, &m->x, B * H)) != SA_OK || (st = dev_alloc(m, &m->x2, B * H)) != SA_OK || (st = dev_alloc(m, &m->h, B * H)) != SA_OK ||
+    if ((st = dev_alloc(m, &m->x, B * H)) != SA_OK || (st = dev_alloc(m, &m->x2, B * H)) != SA_OK ||
+        (st = dev_alloc(m, &m->h, B * H)) != SA_OK ||
         (st = dev_alloc(m, &m->q, B * s.Nq)) != SA_OK || (st = dev_alloc(m, &m->k, B * s.Nk)) != SA_OK ||
         (st = dev_alloc(m, &m->v, B * s.Nk)) != SA_OK || (st = dev_alloc(m, &m->q_rope, B * s.Nq)) != SA_OK ||
         (st = dev_alloc(m, &m->attn, B * s.Nq)) != SA_OK || (st = dev_alloc(m, &m->act, B * s.I)) != SA_OK ||
@@ -841,8 +840,9 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
 
     // Rows [r0, r0 + n) of the batch on one stream: its own split-K partials
     // and decode workspace; x, h, attn and act rows at the same offsets.  At
-    // most kFewRows rows take the few-row launches (few_rows.hip): no norm or
-    // activation launches, the residual stream alternating between x and x2.
+    // most kFewRows rows take the few-row launches (few_rows.hip) except beside
+    // long attention: no norm or activation launches, the residual stream
+    // alternating between x and x2.
     struct Rows {
         int r0, n;
         float* part;
@@ -882,8 +882,9 @@ extern "C" sa_status sa_qwen3_decode_step(sa_qwen3* m, sa_kvcache* cache, const 
     // (A separate split kernel cost 4.7 us per layer.)
     auto attention = [&](Rows& r, int l) {
         const sa_qwen3::Layer& L = m->layers[l];
-        return sa::append_decode_partials(cache, l, r.part, r.few ? 1 : r.beside ? r.gb.qkv.S : r.g.qkv.split, r.n, r.ids.data(), s.Hq, L.q_norm,
-                                          L.k_norm, eps, m->rope_cos, m->rope_sin, d.max_pos, scale,
+        const int n_part = r.few ? 1 : r.beside ? r.gb.qkv.S : r.g.qkv.split;
+        return sa::append_decode_partials(cache, l, r.part, n_part, r.n, r.ids.data(), s.Hq, L.q_norm, L.k_norm, eps,
+                                          m->rope_cos, m->rope_sin, d.max_pos, scale,
                                           m->attn + (size_t)r.r0 * s.Nq, nullptr, r.ws, r.ws_bytes,
                                           l + 1 == d.num_layers ? 1 : 0, r.st, r.few ? &r.parts : nullptr);
     };

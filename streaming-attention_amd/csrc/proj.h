@@ -1,4 +1,5 @@
-// The decoder's projections of more rows than few_rows.hip takes (proj.hip).
+// The decoder's projections of prompts and of decode steps that few_rows.hip does
+// not take (proj.hip).
 #pragma once
 
 #include "sa_internal.h"

@@ -1,4 +1,4 @@
-// The decoder's projections for more than 16 token rows: fp32 rows times bf16
+// The decoder's projections for prompts and larger decode steps: fp32 rows times bf16
 // weights on v_mfma_f32_16x16x32_bf16, every row value as three bf16 terms
 // (bf16_terms.h), so the result is the fp32 product to within 2^-27 of |x|.
 #include "proj.h"

@@ -228,6 +228,9 @@ struct RowPairs {
     }
 };
 
+// Order of a greedy maximum: the larger value, of equal ones the lower index.
+__device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
+
 // Cache rows of the sequences of one launch, passed by value in the kernel
 // arguments (the host has checked every one of them against the page table).
 constexpr int kRowsPerLaunch = 64;
