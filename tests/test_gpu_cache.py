@@ -547,7 +547,7 @@ def append_equals_standalone(sa, d, shift, bf16, S):
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("d", [8, 16, 32, 64, 128, 256])
 def test_append_equals_standalone_norm_rope(sa, d, shift, bf16):
-    """A prompt's append over ragged row counts, from 16-byte aligned pointers
+    """A small append over ragged row counts, from 16-byte aligned pointers
     and from pointers 4 bytes past: the bits of the standalone norm + RoPE."""
     append_equals_standalone(sa, d, shift, bf16, 67)
 

@@ -106,9 +106,10 @@ def test_qk_norm_eps_placement(sa, oracle, synth, eps_outside):
 @pytest.mark.parametrize("M,K,N", [(1, 4, 3), (2, 20, 257), (24, 1028, 3070), (17, 1028, 4100), (33, 516, 6145), (31, 1000, 8190),
                                    (65, 132, 8200), (300, 2052, 1000), (1000, 96, 3000)])
 def test_linear_tiles_and_remainders(sa, synth, M, K, N):
-    """Every tile of the LDS-free kernel (sizes the cost rule gives each of
-    them on 256 CUs), with ragged rows and columns, k ranges that end inside
-    a 32-wide step, fewer steps than waves, and N that takes scalar stores;
+    """The LDS-free kernel's tiles up to 32 x 64 (sizes the cost rule gives each
+    of them on 256 CUs; 64 x 64: test_linear_kernel_of_many_tiles) and the LDS
+    kernel, with ragged rows and columns, k ranges that end inside a 32-wide
+    step, fewer steps than waves, and N that takes scalar stores;
     the rows around the output stay as they were.  fp32 sums in any order are
     within the bars above."""
     x = synth.normal(50, M + K, (M, K))
